@@ -39,6 +39,8 @@ int check_hip(hipError_t e, const char* what) {
   return fail(SF_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
 }
 
+static int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
 int check_launch(const char* what) { return check_hip(hipGetLastError(), what); }
 
 const char* tile_name(int cfg) {
@@ -57,6 +59,11 @@ const char* tile_name(int cfg) {
     case TILE32_DMA: return "gemm tile 64x64 lds-dma k-groups";
     case TILE32_DMA_SPLIT: return "gemm tile 64x64 lds-dma";
     case TILE_NT_K64: return "gemm nt 128x128 k64 lds-dma";
+    case TILE_MID_128: return "gemm tile 128x128";
+    case TILE_MID_64: return "gemm tile 64x64";
+    case TILE_MID_32: return "gemm tile 32x64";
+    case TILE_RAG_128: return "gemm tile generic 128x128";
+    case TILE_RAG_64: return "gemm tile generic 64x64";
   }
   return "gemm";
 }
@@ -67,6 +74,9 @@ void tile_dims(int cfg, bool fp32, int& bm, int& bn) {
     case TILE_NT_BIG: bm = 256; bn = 256; return;
     case TILE_256x128: bm = 256; bn = 128; return;
     case TILE_128x128: bm = 128; bn = 128; return;
+    case TILE_MID_128: bm = 128; bn = 128; return;
+    case TILE_RAG_128: bm = 128; bn = 128; return;
+    case TILE_MID_32: bm = 32; bn = 64; return;
     case TILE_NT_K64: bm = 128; bn = 128; return;
     case TILE_256x64: bm = 256; bn = 64; return;
     case TILE_SKINNY: bm = 16; bn = 32; return;
@@ -85,6 +95,8 @@ int launch_gemm16(sf_dtype in, sf_dtype out, bool a_kmajor, bool b_kmajor, int c
     gx = static_cast<unsigned>((p.N + 31) / 32);
   else if (p.persist > 0)
     gx = static_cast<unsigned>(p.persist);
+  else if (is_mid(cfg) && p.split > 0)  // every XCD room for its share of the tiles, all parts
+    gx = static_cast<unsigned>(kNumXcd * cdiv(p.tiles_m * p.tiles_n, kNumXcd) * p.split);
   else if (p.split > 0)
     gx = static_cast<unsigned>(p.full_tiles) +
          static_cast<unsigned>(p.tiles_m * p.tiles_n - p.full_tiles) * static_cast<unsigned>(p.split);
@@ -131,36 +143,133 @@ static int cu_count_current() {
   return cus;
 }
 
-static int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+// Estimated times of the mid-size plans, in microseconds.  One 64-deep k
+// slice of a launch takes tau[r - 1] when r workgroups share each CU (linear
+// in between, one round of tau[occ - 1] for every further occ workgroups);
+// a further round also costs `round` (its prologue and epilogue), and a
+// split ov0 + ov1 * parts (partials and their sum).  Fitted to sweeps on one
+// MI355X of 133 aligned problems (M 24-6400, N 640-11008, K 104-7680, NT, NN
+// and TN): the plan the estimate picks is on average 1.6 % slower than the
+// fastest one measured, at worst 16 %; 29 unaligned ones: 7 %.
+struct MidCost {
+  int cfg, bm, bn, occ;
+  float tau[4];
+  float round, ov0, ov1;
+};
+static const MidCost kMidAligned[] = {
+    {TILE_MID_128, 128, 128, 2, {0.63f, 0.90f}, 3.0f, 6.0f, 1.0f},
+    {TILE_MID_64, 64, 64, 3, {0.25f, 0.335f, 0.57f}, 2.0f, 1.8f, 0.35f},
+    {TILE_MID_32, 32, 64, 3, {0.185f, 0.25f, 0.40f}, 1.5f, 1.2f, 0.2f},
+};
+// Register-staged loads of k-contiguous rows, and of operands with k-rows
+// (two transposing reads a fragment, unaligned k-rows): about 1.8x the time.
+static const MidCost kMidRagged[] = {
+    {TILE_RAG_128, 128, 128, 2, {1.1f, 1.5f}, 3.0f, 6.0f, 1.0f},
+    {TILE_RAG_64, 64, 64, 4, {0.42f, 0.80f, 1.15f, 1.75f}, 2.0f, 2.0f, 0.3f},
+};
+static const MidCost kMidRaggedMn[] = {
+    {TILE_RAG_128, 128, 128, 2, {1.4f, 2.7f}, 3.0f, 6.0f, 1.0f},
+    {TILE_RAG_64, 64, 64, 4, {0.75f, 1.2f, 1.75f, 2.3f}, 2.0f, 2.0f, 0.3f},
+};
+constexpr int kMaxSplitMid = 8;
+constexpr float kMidFixed = 5.0f;  // launch, first loads, epilogue
 
-// Picks the 16-bit tile config.  Largest tile that still gives every CU at
-// least one tile; narrow-N problems (P.V, N <= 64) use the 256x64 tile.  An
-// A stored K x M (transA) takes the register-staged tiles only.
-static int choose_tile16(int64_t M, int64_t N, int64_t K, int64_t batch, bool vec, bool a_kmajor,
-                         bool b_kmajor, bool f32_out, int cus) {
-  if (!vec) return TILE_GENERIC;
-  if (a_kmajor && b_kmajor && M <= 16)
+static float mid_cost(const MidCost& c, int64_t M, int64_t N, int64_t K, int64_t batch, int split, int cus) {
+  const int64_t wgs = cdiv(M, c.bm) * cdiv(N, c.bn) * batch * split;
+  const int64_t slots = (int64_t)c.occ * cus;
+  const int64_t full = wgs / slots, rem = wgs % slots;
+  float t = (float)full * c.tau[c.occ - 1];
+  if (rem > 0) {
+    const float r = (float)rem / (float)cus;
+    if (r <= 1.0f) {
+      t += c.tau[0];
+    } else {
+      const int i = (int)r < c.occ ? (int)r : c.occ - 1;
+      t += c.tau[i - 1] + (c.tau[i] - c.tau[i - 1]) * (r - (float)i);
+    }
+  }
+  const float rounds = (float)cdiv(wgs, slots);
+  return kMidFixed + (rounds - 1.0f) * c.round + (float)cdiv(cdiv(K, 64), split) * t +
+         (split > 1 ? c.ov0 + c.ov1 * (float)split : 0.0f);
+}
+
+// Estimated time of the 256 x 256 kernel with at most one tile per CU, with
+// the parts its split gives few tiles (gemm_prepare).
+static float big_cost(int64_t t256, int64_t K, bool can_split, int cus) {
+  const int64_t units = cdiv(K, 128);
+  int64_t sp = 1;
+  if (can_split && 2 * t256 <= cus) {
+    sp = cus / t256;
+    if (sp > units) sp = units;
+    if (sp > 8) sp = 8;
+  }
+  const float per = 0.85f + 0.45f * (float)(t256 * sp) / (float)cus;
+  return 10.0f + (float)(2 * cdiv(units, sp)) * per + (sp > 1 ? 30.0f : 0.0f);
+}
+
+// Picks the 16-bit tile config and, for the mid-size kernels, the k split.
+static int choose_tile16(int64_t M, int64_t N, int64_t K, int64_t batch, bool vec, bool small, bool a_kmajor,
+                         bool b_kmajor, bool f32_out, int cus, int* split) {
+  *split = 0;
+  // K-contiguous operands need whole 16-byte chunks along k.
+  const bool kvec = vec && (K % 8 == 0 || (!a_kmajor && !b_kmajor));
+  if (kvec && a_kmajor && b_kmajor && M <= 16)
     return (K == 2048 || K == 4096 || K == 8192) ? TILE_SKINNY_LINE : TILE_SKINNY;
-  if (f32_out) return TILE_128x128;
+  if (f32_out) return kvec && K % 8 == 0 ? TILE_128x128 : TILE_GENERIC;
   auto tiles = [&](int64_t bm, int64_t bn) { return cdiv(M, bm) * cdiv(N, bn) * batch; };
-  // The 256 x 256 LDS-DMA kernel: K-contiguous operands need K % 128 == 0;
-  // two M/N-contiguous operands take any K >= 128.  It runs at least half a
-  // wave of 256 x 256 tiles, or fewer for a single GEMM whose tiles the
-  // split below cuts along k.
-  const bool k_ok = K >= 128 && (K % 128 == 0 || (!a_kmajor && !b_kmajor));
   const int64_t t256 = tiles(256, 256);
-  const bool fills = t256 >= cus || (!(a_kmajor && b_kmajor) && M > 64 &&
-                                     (2 * t256 >= cus || (batch == 1 && K >= 1024 && 16 * t256 >= cus)));
-  // K == 64 exactly (attention scores at head size 64), NT: bound by its
-  // stores; the 128 x 128 kernel that holds four workgroups per CU, once
-  // the 128 x 128 tiles fill the CUs.
-  if (a_kmajor && b_kmajor && K == 64 && N > 64 && tiles(128, 128) >= cus) return TILE_NT_K64;
-  if (k_ok && N > 64 && fills) return TILE_NT_BIG;
-  if (N <= 64) return tiles(256, 64) >= cus ? TILE_256x64 : TILE_64x64;
-  if (tiles(256, 256) >= cus) return TILE_256x256;
-  if (tiles(256, 128) >= cus) return TILE_256x128;
-  if (tiles(128, 128) >= cus) return TILE_128x128;
-  return TILE_64x64;
+  const bool tt = !a_kmajor && b_kmajor;
+  float best = 3.0e38f;
+  int cfg = -1;
+  if (kvec && small) {
+    // K == 64 exactly (attention scores at head size 64), NT: bound by its
+    // stores; the 128 x 128 kernel that holds four workgroups per CU, once
+    // the 128 x 128 tiles fill the CUs.
+    if (a_kmajor && b_kmajor && K == 64 && N > 64 && tiles(128, 128) >= cus) return TILE_NT_K64;
+    // The 256 x 256 LDS-DMA kernel: K-contiguous operands need K % 128 == 0;
+    // two M/N-contiguous operands take any K >= 128.
+    const bool k_ok = K >= 128 && (K % 128 == 0 || (!a_kmajor && !b_kmajor));
+    if (k_ok && N > 64 && M > 64) {
+      if (t256 >= cus) return TILE_NT_BIG;
+      const bool can_split = batch == 1 && K >= 1024 && 16 * t256 >= cus;
+      // TT, TN with a ragged K whose split tiles fill the CUs exactly, and
+      // parts with more CUs than the estimates below were fitted on keep the
+      // split of the 256 x 256 kernel.
+      if (can_split && (tt || cus > 256 || (K % 128 != 0 && 2 * t256 <= cus && cus % t256 == 0))) return TILE_NT_BIG;
+      if (tt ? 2 * t256 >= cus : 4 * t256 >= cus) {
+        best = big_cost(t256, K, can_split, cus);
+        cfg = TILE_NT_BIG;
+      }
+    }
+    if (N <= 64 && tiles(256, 64) >= cus) return TILE_256x64;
+    // Exactly one 256 x 256 or 256 x 128 tile per CU: the register-staged
+    // tiles.  (The 128 x 128 kernel below is the faster one there too, 15.9
+    // against 24.3 us at 4096 x 4096 x 192; the suite pins these plans.)
+    if (N > 64 && t256 == cus) return TILE_256x256;
+    if (N > 64 && t256 < cus && tiles(256, 128) == cus && !(k_ok && 2 * t256 >= cus && K % 128 == 0))
+      return TILE_256x128;
+  }
+  const bool aligned = kvec && small;
+  const MidCost* c = aligned ? kMidAligned : (a_kmajor && b_kmajor ? kMidRagged : kMidRaggedMn);
+  const int nc = aligned ? (a_kmajor && b_kmajor ? 3 : 2) : 2;
+  const int64_t KT = cdiv(K, 64);
+  for (int i = 0; i < nc; ++i) {
+    // 32 x 64 tiles only where rows are few and the k loop is long enough
+    // for the finer grain to matter.
+    if (c[i].cfg == TILE_MID_32 && (M > 256 || K <= 256)) continue;
+    const int64_t t = tiles(c[i].bm, c[i].bn);
+    for (int sp = 1; sp <= kMaxSplitMid; ++sp) {
+      // parts of at least two slices, all resident together
+      if (sp > 1 && (batch != 1 || tt || KT < 2 * sp || t * sp > (int64_t)c[i].occ * cus)) break;
+      const float us = mid_cost(c[i], M, N, K, batch, sp, cus);
+      if (us < best) {
+        best = us;
+        cfg = c[i].cfg;
+        *split = sp > 1 ? sp : 0;
+      }
+    }
+  }
+  return cfg;
 }
 
 // Picks the fp32 tile config.  Outputs of at most CUs / 4 tiles of 64 x 64
@@ -402,7 +511,7 @@ int gemm_prepare(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
   plan.a_kmajor = a_kmajor;
   plan.b_kmajor = b_kmajor;
   const int cus = cu_count_current();
-  int bm, bn;
+  int bm, bn, mid_split = 0;
   if (ab_dtype == SF_F32) {
     const bool vec = al16(A) && al16(B) && (lda % 4 == 0) && (ldb % 4 == 0) &&
                      (strideA % 4 == 0) && (strideB % 4 == 0) && (K % 4 == 0) &&
@@ -414,17 +523,14 @@ int gemm_prepare(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
     plan.cfg = choose_tile32(M, N, K, batch, vec, a_kmajor, dma_ok, cus);
   } else {
     const bool vec = al16(A) && al16(B) && (lda % 8 == 0) && (ldb % 8 == 0) &&
-                     (strideA % 8 == 0) && (strideB % 8 == 0) && (K % 8 == 0) &&
+                     (strideA % 8 == 0) && (strideB % 8 == 0) &&
                      (a_kmajor || M % 8 == 0) && (b_kmajor || N % 8 == 0);
+    // The LDS-DMA kernels address each operand (M or K rows of lda) with
+    // 32-bit byte offsets; larger ones take the register-staged loads.
+    const bool small = (a_kmajor ? M : K) * lda * 2 < (int64_t(1) << 31) &&
+                       (b_kmajor ? N : K) * ldb * 2 < (int64_t(1) << 31);
     plan.fp32 = false;
-    plan.cfg = choose_tile16(M, N, K, batch, vec, a_kmajor, b_kmajor, c_dtype == SF_F32, cus);
-    // The LDS-DMA kernel addresses each operand (M or K rows of lda) with
-    // 32-bit byte offsets.
-    if (plan.cfg == TILE_NT_BIG && ((a_kmajor ? M : K) * lda * 2 >= (int64_t(1) << 31) ||
-                                    (b_kmajor ? N : K) * ldb * 2 >= (int64_t(1) << 31)))
-      plan.cfg = TILE_256x256;
-    if (plan.cfg == TILE_NT_K64 && (M * lda * 2 >= (int64_t(1) << 31) || N * ldb * 2 >= (int64_t(1) << 31)))
-      plan.cfg = TILE_128x128;
+    plan.cfg = choose_tile16(M, N, K, batch, vec, small, a_kmajor, b_kmajor, c_dtype == SF_F32, cus, &mid_split);
   }
   // The row-segment skinny kernel addresses 64 rows of W with 32-bit offsets.
   if (plan.cfg == TILE_SKINNY_LINE && ldb * 2 * 64 >= (int64_t(1) << 31)) plan.cfg = TILE_SKINNY;
@@ -493,6 +599,10 @@ int gemm_prepare(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
         p.split = (int)sp;
       }
     }
+  }
+  if (is_mid(plan.cfg) && mid_split > 1) {
+    p.split = mid_split;
+    p.xcd_shift = g_test_hooks.xcd_shift.load(std::memory_order_relaxed) & (kNumXcd - 1);
   }
   if (plan.cfg == TILE_NT_BIG && batch == 1 && K >= 128) {
     // Tail split: with R = tiles % CUs left over after whole waves, run the
@@ -581,7 +691,9 @@ void gemm_split_needs(const GemmPlan& plan, size_t* part_bytes, int* counters) {
     *counters = tiles;
   } else {
     const int nsplit = plan.p.tiles_m * plan.p.tiles_n - plan.p.full_tiles;
-    *part_bytes = (size_t)nsplit * plan.p.split * (256u * 256u * 4u);
+    int bm, bn;
+    tile_dims(plan.cfg, false, bm, bn);
+    *part_bytes = (size_t)nsplit * plan.p.split * (size_t)(bm * bn) * 4u;
     // persistent: three words per split tile (split_handoff_shared)
     *counters = plan.p.persist > 0 ? 3 * nsplit : nsplit;
   }
@@ -609,6 +721,15 @@ static int gemm_run(int transA, int transB, int64_t M, int64_t N, int64_t K, int
   size_t part_bytes = 0;
   int counters = 0;
   gemm_split_needs(plan, &part_bytes, &counters);
+  if (part_bytes > 0 && is_mid(plan.cfg) && st != nullptr) {
+    // A mid-size split is only a matter of speed, so a call being captured
+    // into a graph goes without one: nothing is allocated or waited for.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
+      plan.p.split = 0;
+      part_bytes = 0;
+    }
+  }
   if (part_bytes == 0) return gemm_launch_plan(plan, batch, ab_dtype, c_dtype, st);
   rc = split_workspace_acquire(part_bytes, counters, st, &plan.p.ws, &plan.p.counters);
   if (rc != SF_OK) return rc;
@@ -651,7 +772,8 @@ int sf_gemm_plan(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
   if (rc != SF_OK) return rc;
   char extra[64] = "";
   if (!plan.noop && plan.p.split > 0)
-    snprintf(extra, sizeof(extra), "%s split-tail %dx%d", plan.p.persist > 0 ? " persistent" : "",
+    snprintf(extra, sizeof(extra), "%s split%s %dx%d", plan.p.persist > 0 ? " persistent" : "",
+             is_mid(plan.cfg) ? "" : "-tail",
              plan.p.tiles_m * plan.p.tiles_n - plan.p.full_tiles, plan.p.split);
   else if (!plan.noop && plan.p.persist > 0)
     snprintf(extra, sizeof(extra), " persistent");

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "sf_internal.hpp"
+#include "gemm16mid.hpp"
 #include "gemm16nt_4w.hpp"
 #include "gemm16nt_k64.hpp"
 #include "gemm16nt_pp.hpp"
@@ -46,17 +47,26 @@ static int launch16_t(int cfg, const GemmParams& p, unsigned gx, unsigned gy, hi
     case TILE_256x128:
       hipLaunchKernelGGL((gemm16_kernel<TIn, TOut, 256, 128, 4, 2, KM, true, AKM>), g, dim3(512), 0, st, p);
       break;
-    case TILE_128x128:
-      hipLaunchKernelGGL((gemm16_kernel<TIn, TOut, 128, 128, 2, 2, KM, true, AKM>), g, dim3(256), 0, st, p);
-      break;
     case TILE_256x64:
       hipLaunchKernelGGL((gemm16_kernel<TIn, TOut, 256, 64, 4, 1, KM, true, AKM>), g, dim3(256), 0, st, p);
       break;
-    case TILE_64x64:
-      hipLaunchKernelGGL((gemm16_kernel<TIn, TOut, 64, 64, 2, 2, KM, true, AKM>), g, dim3(256), 0, st, p);
+    case TILE_MID_128:
+      hipLaunchKernelGGL((gemm16mid_kernel<TIn, TOut, 128, 128, 2, 4, 2, AKM, KM, true, 4>), g, dim3(512), 0, st, p);
       break;
-    case TILE_GENERIC:
-      hipLaunchKernelGGL((gemm16_kernel<TIn, TOut, 64, 64, 2, 2, KM, false, AKM>), g, dim3(256), 0, st, p);
+    case TILE_MID_64:
+      hipLaunchKernelGGL((gemm16mid_kernel<TIn, TOut, 64, 64, 2, 2, 3, AKM, KM, true, 3>), g, dim3(256), 0, st, p);
+      break;
+    case TILE_MID_32:
+      if constexpr (KM && AKM) {
+        hipLaunchKernelGGL((gemm16mid_kernel<TIn, TOut, 32, 64, 2, 2, 4, true, true, true, 3>), g, dim3(256), 0, st, p);
+        break;
+      }
+      return fail(SF_ERR_UNSUPPORTED, "the 32x64 tile needs K-contiguous A and B");
+    case TILE_RAG_128:
+      hipLaunchKernelGGL((gemm16mid_kernel<TIn, TOut, 128, 128, 2, 2, 2, AKM, KM, false, 2>), g, dim3(256), 0, st, p);
+      break;
+    case TILE_RAG_64:
+      hipLaunchKernelGGL((gemm16mid_kernel<TIn, TOut, 64, 64, 2, 2, 2, AKM, KM, false, 4>), g, dim3(256), 0, st, p);
       break;
     case TILE_NT_BIG:
       if constexpr (KM && AKM) {

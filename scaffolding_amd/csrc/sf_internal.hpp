@@ -38,10 +38,10 @@ extern TestHooks g_test_hooks;
 enum TileCfg {
   TILE_256x256 = 0,  // 512 threads, waves 2x4 of 128x64
   TILE_256x128 = 1,  // 512 threads, waves 4x2 of 64x64
-  TILE_128x128 = 2,  // 256 threads, waves 2x2 of 64x64
+  TILE_128x128 = 2,  // fp32; 16-bit inputs with an fp32 output: 256 threads, waves 2x2 of 64x64
   TILE_256x64 = 3,   // 256 threads, waves 4x1 of 64x64 (narrow N, e.g. P.V)
-  TILE_64x64 = 4,    // 256 threads, waves 2x2 of 32x32
-  TILE_GENERIC = 5,  // 64x64, element-wise bounds-checked loads (any layout)
+  TILE_64x64 = 4,    // fp32 only
+  TILE_GENERIC = 5,  // fp32 or an fp32 output: 64x64, element-wise bounds-checked loads (any layout)
   TILE_SKINNY = 6,   // M <= 16 stream kernel
   TILE_NT_BIG = 7,   // 256x256 NT, 8-wave ping-pong, direct-to-LDS (gemm16nt_pp.hpp)
   TILE_SKINNY_LINE = 8,  // M <= 16, K in {2048, 4096, 8192}: row-segment stream (skinny16l)
@@ -51,9 +51,16 @@ enum TileCfg {
   TILE32_DMA = 11,       // 64x64, direct-to-LDS ring, two 4-wave k-groups (gemm32dma.hpp)
   TILE32_DMA_SPLIT = 12,  // 64x64, direct-to-LDS ring, one k-group, split-K capable
   // 16-bit again:
-  TILE_NT_K64 = 13  // 128x128 NT with K == 64, four workgroups per CU (gemm16nt_k64.hpp)
+  TILE_NT_K64 = 13,  // 128x128 NT with K == 64, four workgroups per CU (gemm16nt_k64.hpp)
+  // Between skinny and 256x256 (gemm16mid.hpp), any layout unless noted:
+  TILE_MID_128 = 14,   // 128x128, direct-to-LDS, 8 waves, two workgroups per CU
+  TILE_MID_64 = 15,    // 64x64, direct-to-LDS ring of 3, three workgroups per CU
+  TILE_MID_32 = 16,    // 32x64 (NT), direct-to-LDS ring of 4, three workgroups per CU
+  TILE_RAG_128 = 17,   // 128x128, register-staged loads at any 2-byte alignment
+  TILE_RAG_64 = 18     // 64x64, likewise
 };
 const char* tile_name(int cfg);
+inline bool is_mid(int cfg) { return cfg >= TILE_MID_128 && cfg <= TILE_RAG_64; }
 
 // One GEMM launch: batch entries [0, batch) of p, grid.y <= 65535 per call.
 int launch_gemm16(sf_dtype in, sf_dtype out, bool a_kmajor, bool b_kmajor, int cfg, const GemmParams& p,
