@@ -257,6 +257,26 @@ int sf_attention_heads(const void* Q, int64_t ldq, int64_t strideQ, int64_t head
                        int64_t batch, int64_t heads, int64_t Sq, int64_t Sk, int64_t D,
                        float scale, sf_dtype dtype, void* stream);
 
+/* sf_attention_heads for head sizes up to 128 and with an additive mask:
+ *   O[b,h] = softmax(scale * Q K^T + mask) V,
+ *   mask element (b, h, i, j) at mask + b * mask_batch + h * mask_head
+ *   + i * mask_row + j  (element strides >= 0; 0 broadcasts over that axis)
+ * of dtype `dtype` or F32 at its natural alignment; NULL for none (the
+ * mask_* arguments are then ignored).  -inf entries drop a key; a row of
+ * -inf only gives NaN and a row of the type's lowest value only gives the
+ * mean of V, as softmax(scores + mask) does.  fp32 scores, mask sum and
+ * softmax.  D a multiple of 8 up to 128; the other rules and errors are
+ * sf_attention_heads'.  Replaces the masked branch of
+ * scaled_dot_product_attention (nn/functional.py:339-347) as well. */
+int sf_attention_masked(const void* Q, int64_t ldq, int64_t strideQ, int64_t headQ,
+                        const void* K, int64_t ldk, int64_t strideK, int64_t headK,
+                        const void* V, int64_t ldv, int64_t strideV, int64_t headV,
+                        void* O, int64_t ldo, int64_t strideO, int64_t headO,
+                        int64_t batch, int64_t heads, int64_t Sq, int64_t Sk, int64_t D,
+                        float scale, sf_dtype dtype,
+                        const void* mask, sf_dtype mask_dtype,
+                        int64_t mask_batch, int64_t mask_head, int64_t mask_row, void* stream);
+
 /* Layer normalisation of `rows` contiguous rows of `cols` elements, with an
  * optional per-group affine modulation (adaptive layer norm):
  *   mu = mean(x[r,:]),  var = mean((x[r,:] - mu)^2)  (population variance)

@@ -87,6 +87,13 @@ cdef extern from "sfgemm.h" nogil:
                            void* O, int64_t ldo, int64_t strideO, int64_t headO,
                            int64_t batch, int64_t heads, int64_t Sq, int64_t Sk, int64_t D,
                            float scale, sf_dtype dtype, void* stream)
+    int sf_attention_masked(const void* Q, int64_t ldq, int64_t strideQ, int64_t headQ,
+                            const void* K, int64_t ldk, int64_t strideK, int64_t headK,
+                            const void* V, int64_t ldv, int64_t strideV, int64_t headV,
+                            void* O, int64_t ldo, int64_t strideO, int64_t headO,
+                            int64_t batch, int64_t heads, int64_t Sq, int64_t Sk, int64_t D,
+                            float scale, sf_dtype dtype, const void* mask, sf_dtype mask_dtype,
+                            int64_t mask_batch, int64_t mask_head, int64_t mask_row, void* stream)
     int sf_layer_norm(const void* x, void* y, int64_t rows, int64_t cols,
                       const void* gamma, const void* beta, float eps,
                       const void* mod_scale, const void* mod_shift, int64_t mod_ld, int64_t group_rows,
@@ -1013,10 +1020,10 @@ cdef object _mha_strided(q, int64_t q_off, int64_t ldq, k, int64_t k_off, int64_
     cdef char* pv = <char*>_ptr(v) + v_off * es
     cdef char* po = <char*>_ptr(out)
     cdef int ret = SF_ERR_UNSUPPORTED
-    if sdt != SF_F32 and 8 <= D <= 64 and D % 8 == 0 and scale > 0:
+    if sdt != SF_F32 and 8 <= D <= 128 and D % 8 == 0 and scale > 0:
         with nogil:
-            ret = sf_attention_heads(pq, ldq, Nq * ldq, D, pk, ldk, Sk * ldk, D, pv, ldv, Sk * ldv, D,
-                                     po, C, Nq * C, D, B, H, Nq, Sk, D, scale, sdt, NULL)
+            ret = sf_attention_masked(pq, ldq, Nq * ldq, D, pk, ldk, Sk * ldk, D, pv, ldv, Sk * ldv, D,
+                                      po, C, Nq * C, D, B, H, Nq, Sk, D, scale, sdt, NULL, sdt, 0, 0, 0, NULL)
         if ret != SF_ERR_UNSUPPORTED:
             _check_kernel(ret)
             return out
@@ -1218,19 +1225,25 @@ def _mask_layout(tuple mshape, tuple sshape):
     return per, merged[1][0], merged[0][1], merged[1][1], s_row, s_col
 
 
+cdef object _device_mask(mask, gt):
+    """`mask` on gt's device, fp32 or of gt's dtype."""
+    if not isinstance(mask, GpuTensor):
+        mask = gputensor_from_numpy(np.ascontiguousarray(mask, dtype=np.float32), gt.device_id)
+    if mask.device_id != gt.device_id:
+        raise ValueError("dev_softmax_masked: the mask is on device %d, the scores on %d"
+                         % (mask.device_id, gt.device_id))
+    if mask.dtype != np.float32 and mask.dtype != gt.dtype:
+        mask = dev_cast(mask, np.float32)
+    return mask
+
+
 def dev_softmax_masked(scores, mask, float scale=1.0):
     """softmax(scale * scores + mask) along the last dim, in place of the
     reference's host branch scores *= scale; scores += mask; softmax
     (nn/functional.py:337-347).  `mask` (a GpuTensor, or a host array that
     is uploaded as fp32) broadcasts to the scores' shape with NumPy's rules;
     additive, -inf entries allowed."""
-    if not isinstance(mask, GpuTensor):
-        mask = gputensor_from_numpy(np.ascontiguousarray(mask, dtype=np.float32), scores.device_id)
-    if mask.device_id != scores.device_id:
-        raise ValueError("dev_softmax_masked: the mask is on device %d, the scores on %d"
-                         % (mask.device_id, scores.device_id))
-    if mask.dtype != np.float32 and mask.dtype != scores.dtype:
-        mask = dev_cast(mask, np.float32)
+    mask = _device_mask(mask, scores)
     sshape = tuple(scores.shape)
     if len(sshape) == 0:
         raise ValueError("dev_softmax_masked: scalar input")
@@ -1278,9 +1291,9 @@ def dev_scaled_dot_product_attention(q, k, v, scale=None, attn_mask=None, float 
     """softmax(scale * Q K^T (+ attn_mask)) V  (reference GPU path
     nn/functional.py:310-321; the mask as its host branch :339-341).
     q (..., Sq, D), k and v (..., Sk, D) with equal leading dims.  One fused
-    launch (sf_attention: scores never reach memory) for 16-bit inputs with
-    D a multiple of 8 up to 64, a positive finite scale, no mask and no
-    dropout; otherwise, or when sf_attention declines the call
+    launch (sf_attention_masked: scores never reach memory) for 16-bit inputs
+    with D a multiple of 8 up to 128, a positive finite scale and no dropout;
+    otherwise, or when sf_attention_masked declines the call
     (SF_ERR_UNSUPPORTED), the three-launch path (dropout_p > 0: dev_dropout
     on the probabilities with the stream (seed, offset))."""
     d = q.shape[-1]
@@ -1300,9 +1313,22 @@ def dev_scaled_dot_product_attention(q, k, v, scale=None, attn_mask=None, float 
         batch *= e
     if not (0.0 <= dropout_p < 1.0):
         raise ValueError("dev_scaled_dot_product_attention: dropout_p must be in [0, 1), got %r" % dropout_p)
-    if attn_mask is not None or dropout_p > 0.0 or q.dtype == np.float32 or d < 8 or d > 64 or d % 8 != 0 \
-            or not (0.0 < s < 3.0e38):
+    if dropout_p > 0.0 or q.dtype == np.float32 or d < 8 or d > 128 or d % 8 != 0 or not (0.0 < s < 3.0e38):
         return dev_sdpa_unfused(q, k, v, scale, attn_mask, dropout_p, seed, offset)
+    # The mask's broadcast over the leading dims, as an outer and an inner
+    # group of them (batch entries and heads of the fused kernel).
+    cdef void* pm = NULL
+    cdef sf_dtype mdt = SF_F32
+    cdef int64_t inner = batch if batch > 0 else 1
+    cdef int64_t m_outer = 0, m_inner = 0, m_row = 0
+    if attn_mask is not None:
+        attn_mask = _device_mask(attn_mask, q)
+        _, c_inner, c_outer, c_in, c_row, c_col = _mask_layout(tuple(attn_mask.shape), tuple(q.shape[:-1]) + (sk,))
+        if c_col == 0:  # one value per row: not the fused kernel's layout
+            return dev_sdpa_unfused(q, k, v, scale, attn_mask)
+        inner, m_outer, m_inner, m_row = c_inner, c_outer, c_in, c_row
+        pm = _ptr(attn_mask)
+        mdt = _sf_dtype(attn_mask.dtype)
     out = _alloc_like(tuple(q.shape), q.dtype, q.device_id)
     cdef int ret
     cdef void* pq = _ptr(q)
@@ -1312,12 +1338,14 @@ def dev_scaled_dot_product_attention(q, k, v, scale=None, attn_mask=None, float 
     cdef sf_dtype dt = _sf_dtype(q.dtype)
     cdef float fs = s
     cdef int64_t dh = d
+    cdef int64_t outer = batch // inner
     with nogil:
-        ret = sf_attention(pq, dh, sq * dh, pk, dh, sk * dh, pv, dh, sk * dh, po, dh, sq * dh,
-                           batch, sq, sk, dh, fs, dt, NULL)
+        ret = sf_attention_masked(pq, dh, inner * sq * dh, sq * dh, pk, dh, inner * sk * dh, sk * dh,
+                                  pv, dh, inner * sk * dh, sk * dh, po, dh, inner * sq * dh, sq * dh,
+                                  outer, inner, sq, sk, dh, fs, dt, pm, mdt, m_outer, m_inner, m_row, NULL)
     if ret == SF_ERR_UNSUPPORTED:
         del out
-        return dev_sdpa_unfused(q, k, v, scale)
+        return dev_sdpa_unfused(q, k, v, scale, attn_mask)
     _check_kernel(ret)
     return out
 

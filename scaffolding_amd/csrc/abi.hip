@@ -242,12 +242,11 @@ static int choose_tile16(int64_t M, int64_t N, int64_t K, int64_t batch, bool ve
       }
     }
     if (N <= 64 && tiles(256, 64) >= cus) return TILE_256x64;
-    // Exactly one 256 x 256 or 256 x 128 tile per CU: the register-staged
-    // tiles.  (The 128 x 128 kernel below is the faster one there too, 15.9
+    // Exactly one 256 x 256 tile per CU, or with K < 256 one 256 x 128: the
+    // register-staged tiles.  (The 128 x 128 kernel below is the faster one there too, 15.9
     // against 24.3 us at 4096 x 4096 x 192; the suite pins these plans.)
     if (N > 64 && t256 == cus) return TILE_256x256;
-    if (N > 64 && t256 < cus && tiles(256, 128) == cus && !(k_ok && 2 * t256 >= cus && K % 128 == 0))
-      return TILE_256x128;
+    if (N > 64 && K < 256 && tiles(256, 128) == cus && cfg < 0) return TILE_256x128;
   }
   const bool aligned = kvec && small;
   const MidCost* c = aligned ? kMidAligned : (a_kmajor && b_kmajor ? kMidRagged : kMidRaggedMn);
@@ -804,54 +803,107 @@ static bool attn_out_disjoint(int64_t S, int64_t ld, int64_t sB, int64_t sH, int
   return B <= 1 || sB >= span;
 }
 
-int sf_attention_heads(const void* Q, int64_t ldq, int64_t strideQ, int64_t headQ, const void* K, int64_t ldk,
-                       int64_t strideK, int64_t headK, const void* V, int64_t ldv, int64_t strideV, int64_t headV,
-                       void* O, int64_t ldo, int64_t strideO, int64_t headO, int64_t batch, int64_t heads,
-                       int64_t Sq, int64_t Sk, int64_t D, float scale, sf_dtype dtype, void* stream) {
+// Validates a fused attention call and fills the shape; SF_OK with *noop for
+// an empty one.  dmax: the largest head size the caller's kernels take.
+static int attn_prepare(const char* name, const void* Q, int64_t ldq, int64_t strideQ, int64_t headQ, const void* K,
+                        int64_t ldk, int64_t strideK, int64_t headK, const void* V, int64_t ldv, int64_t strideV,
+                        int64_t headV, void* O, int64_t ldo, int64_t strideO, int64_t headO, int64_t batch,
+                        int64_t heads, int64_t Sq, int64_t Sk, int64_t D, int64_t dmax, float scale, sf_dtype dtype,
+                        AttnShape& a, bool* noop) {
   g_err[0] = 0;
-  if (!valid_dtype(dtype)) return fail(SF_ERR_INVALID_ARG, "sf_attention: unknown dtype %d", (int)dtype);
-  if (batch < 0 || heads < 0 || Sq < 0 || Sk < 0 || D < 0)
-    return fail(SF_ERR_INVALID_ARG, "sf_attention: negative size");
-  if (dtype == SF_F32) return fail(SF_ERR_UNSUPPORTED, "sf_attention: 16-bit dtypes only");
-  if (D < 8 || D > 64 || D % 8 != 0)
-    return fail(SF_ERR_UNSUPPORTED, "sf_attention: head size %lld (multiples of 8 up to 64)", (long long)D);
+  *noop = false;
+  if (!valid_dtype(dtype)) return fail(SF_ERR_INVALID_ARG, "%s: unknown dtype %d", name, (int)dtype);
+  if (batch < 0 || heads < 0 || Sq < 0 || Sk < 0 || D < 0) return fail(SF_ERR_INVALID_ARG, "%s: negative size", name);
+  if (dtype == SF_F32) return fail(SF_ERR_UNSUPPORTED, "%s: 16-bit dtypes only", name);
+  if (D < 8 || D > dmax || D % 8 != 0)
+    return fail(SF_ERR_UNSUPPORTED, "%s: head size %lld (multiples of 8 up to %lld)", name, (long long)D,
+                (long long)dmax);
   if (!(scale > 0.0f) || scale > 3.0e38f)
-    return fail(SF_ERR_UNSUPPORTED, "sf_attention: scale %g (positive and finite only)", (double)scale);
-  if (batch == 0 || heads == 0 || Sq == 0) return SF_OK;
-  if (Sk == 0) return fail(SF_ERR_INVALID_ARG, "sf_attention: softmax over zero keys");
+    return fail(SF_ERR_UNSUPPORTED, "%s: scale %g (positive and finite only)", name, (double)scale);
+  if (batch == 0 || heads == 0 || Sq == 0) {
+    *noop = true;
+    return SF_OK;
+  }
+  if (Sk == 0) return fail(SF_ERR_INVALID_ARG, "%s: softmax over zero keys", name);
   if (Q == nullptr || K == nullptr || V == nullptr || O == nullptr)
-    return fail(SF_ERR_INVALID_ARG, "sf_attention: null pointer");
+    return fail(SF_ERR_INVALID_ARG, "%s: null pointer", name);
   if (ldq < D || ldk < D || ldv < D || ldo < D)
-    return fail(SF_ERR_INVALID_ARG, "sf_attention: row stride below the head size");
+    return fail(SF_ERR_INVALID_ARG, "%s: row stride below the head size", name);
   if (strideQ < 0 || strideK < 0 || strideV < 0 || strideO < 0 || headQ < 0 || headK < 0 || headV < 0 ||
       headO < 0)
-    return fail(SF_ERR_INVALID_ARG, "sf_attention: negative batch or head stride");
+    return fail(SF_ERR_INVALID_ARG, "%s: negative batch or head stride", name);
   if (!attn_out_disjoint(Sq, ldo, strideO, headO, batch, heads, D))
-    return fail(SF_ERR_INVALID_ARG, "sf_attention: output (batch, head) entries overlap");
+    return fail(SF_ERR_INVALID_ARG, "%s: output (batch, head) entries overlap", name);
   // Key rows up to the next multiple of 64 past Sk are addressed (and read
   // as zeros) with 32-bit offsets.
   if (Sq > INT32_MAX || heads > INT32_MAX || (Sk + 64) * (ldk > ldv ? ldk : ldv) * 2 >= (int64_t(1) << 31))
-    return fail(SF_ERR_UNSUPPORTED, "sf_attention: K/V of one batch entry must stay below 2 GiB");
+    return fail(SF_ERR_UNSUPPORTED, "%s: K/V of one batch entry must stay below 2 GiB", name);
   if (!al16(Q) || !al16(K) || !al16(V) || !al16(O) || ldq % 8 || ldk % 8 || ldv % 8 || ldo % 8 ||
       strideQ % 8 || strideK % 8 || strideV % 8 || strideO % 8 || headQ % 8 || headK % 8 || headV % 8 ||
       headO % 8)
-    return fail(SF_ERR_UNSUPPORTED, "sf_attention: rows must be 16-byte aligned");
-  AttnShape a;
+    return fail(SF_ERR_UNSUPPORTED, "%s: rows must be 16-byte aligned", name);
   a.Q = Q; a.K = K; a.V = V; a.O = O;
   a.ldq = ldq; a.ldk = ldk; a.ldv = ldv; a.ldo = ldo;
   a.sQ = strideQ; a.sK = strideK; a.sV = strideV; a.sO = strideO;
   a.hQ = headQ; a.hK = headK; a.hV = headV; a.hO = headO;
   a.batch = batch; a.heads = heads; a.Sq = Sq; a.Sk = Sk;
   a.D = D;
+  return SF_OK;
+}
+
+int sf_attention_heads(const void* Q, int64_t ldq, int64_t strideQ, int64_t headQ, const void* K, int64_t ldk,
+                       int64_t strideK, int64_t headK, const void* V, int64_t ldv, int64_t strideV, int64_t headV,
+                       void* O, int64_t ldo, int64_t strideO, int64_t headO, int64_t batch, int64_t heads,
+                       int64_t Sq, int64_t Sk, int64_t D, float scale, sf_dtype dtype, void* stream) {
+  AttnShape a;
+  bool noop;
+  int rc = attn_prepare("sf_attention", Q, ldq, strideQ, headQ, K, ldk, strideK, headK, V, ldv, strideV, headV, O,
+                        ldo, strideO, headO, batch, heads, Sq, Sk, D, 64, scale, dtype, a, &noop);
+  if (rc != SF_OK || noop) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const AttnSplit sp = attn_split_plan(a, cu_count_current());
   if (sp.parts == 0) return launch_attention(a, scale, dtype, sp, nullptr, st);
   float* ws = nullptr;
   int* cnt = nullptr;
-  int rc = split_workspace_acquire((size_t)(sp.items - sp.full) * (size_t)sp.parts * kAttnPartBytes, 0, st, &ws,
-                                   &cnt);
+  rc = split_workspace_acquire((size_t)(sp.items - sp.full) * (size_t)sp.parts * kAttnPartBytes, 0, st, &ws, &cnt);
   if (rc != SF_OK) return rc;
   rc = launch_attention(a, scale, dtype, sp, ws, st);
+  const int rc2 = split_workspace_release(st);
+  return rc != SF_OK ? rc : rc2;
+}
+
+int sf_attention_masked(const void* Q, int64_t ldq, int64_t strideQ, int64_t headQ, const void* K, int64_t ldk,
+                        int64_t strideK, int64_t headK, const void* V, int64_t ldv, int64_t strideV, int64_t headV,
+                        void* O, int64_t ldo, int64_t strideO, int64_t headO, int64_t batch, int64_t heads,
+                        int64_t Sq, int64_t Sk, int64_t D, float scale, sf_dtype dtype, const void* mask,
+                        sf_dtype mask_dtype, int64_t mask_batch, int64_t mask_head, int64_t mask_row,
+                        void* stream) {
+  if (mask == nullptr && D <= 64)
+    return sf_attention_heads(Q, ldq, strideQ, headQ, K, ldk, strideK, headK, V, ldv, strideV, headV, O, ldo, strideO,
+                              headO, batch, heads, Sq, Sk, D, scale, dtype, stream);
+  AttnShape a;
+  bool noop;
+  int rc = attn_prepare("sf_attention_masked", Q, ldq, strideQ, headQ, K, ldk, strideK, headK, V, ldv, strideV, headV,
+                        O, ldo, strideO, headO, batch, heads, Sq, Sk, D, 128, scale, dtype, a, &noop);
+  if (rc != SF_OK) return rc;
+  AttnMask m = {mask, mask_dtype, mask_batch, mask_head, mask_row};
+  if (mask != nullptr) {
+    if (!valid_dtype(mask_dtype)) return fail(SF_ERR_INVALID_ARG, "sf_attention_masked: unknown mask dtype");
+    if (mask_dtype != dtype && mask_dtype != SF_F32)
+      return fail(SF_ERR_UNSUPPORTED, "sf_attention_masked: the mask's dtype must be the operands' dtype or F32");
+    if (mask_batch < 0 || mask_head < 0 || mask_row < 0)
+      return fail(SF_ERR_INVALID_ARG, "sf_attention_masked: negative mask stride");
+  }
+  if (noop) return SF_OK;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const AttnSplit sp = attn_wide_split_plan(a, cu_count_current());
+  if (sp.parts == 0) return launch_attention_wide(a, m, scale, dtype, sp, nullptr, st);
+  float* ws = nullptr;
+  int* cnt = nullptr;
+  rc = split_workspace_acquire((size_t)(sp.items - sp.full) * (size_t)sp.parts * attn_wide_part_bytes(D), 0, st, &ws,
+                               &cnt);
+  if (rc != SF_OK) return rc;
+  rc = launch_attention_wide(a, m, scale, dtype, sp, ws, st);
   const int rc2 = split_workspace_release(st);
   return rc != SF_OK ? rc : rc2;
 }

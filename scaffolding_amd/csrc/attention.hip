@@ -5,11 +5,15 @@
 namespace sf {
 
 AttnSplit attn_split_plan(const AttnShape& a, int cus) {
+  return attn_split_items(a.batch * a.heads * ((a.Sq + 255) / 256), a.Sk, kAttnPartBytes, cus);
+}
+
+AttnSplit attn_split_items(int64_t items, int64_t Sk, size_t part_bytes, int cus) {
   AttnSplit sp;
-  sp.items = a.batch * a.heads * ((a.Sq + 255) / 256);
+  sp.items = items;
   sp.full = sp.items;
   sp.parts = 0;
-  const int64_t nb = (a.Sk + 63) / 64;
+  const int64_t nb = (Sk + 63) / 64;
   // Two workgroups per CU, all equally long: the items past the last whole
   // round of slots (the tail) run alone.  They are split into P key ranges
   // (at least 8 key blocks a part, at most 16 parts) when that shortens
@@ -41,7 +45,7 @@ AttnSplit attn_split_plan(const AttnShape& a, int cus) {
   if (tp >= 2) {
     int64_t hp = tp > 16 ? 16 : tp;
     if (hp > nb) hp = nb;
-    const int64_t fit = (int64_t(1) << 30) / ((int64_t)kAttnPartBytes * sp.items);
+    const int64_t fit = (int64_t(1) << 30) / ((int64_t)part_bytes * sp.items);
     if (hp > fit) hp = fit;
     if (hp >= 2) {
       sp.full = 0;
@@ -56,20 +60,25 @@ AttnSplit attn_split_plan(const AttnShape& a, int cus) {
   return sp;
 }
 
-int launch_attention(const AttnShape& a, float scale, sf_dtype dt, const AttnSplit& sp, float* ws, hipStream_t st) {
-  AttnParams p;
+void attn_fill_params(const AttnShape& a, float scale, const AttnSplit& sp, float* ws, int rows, AttnParams& p) {
   p.Q = a.Q; p.K = a.K; p.V = a.V; p.O = a.O;
   p.sQ = a.sQ; p.sK = a.sK; p.sV = a.sV; p.sO = a.sO;
   p.hQ = a.hQ; p.hK = a.hK; p.hV = a.hV; p.hO = a.hO;
+  p.item0 = 0;
   p.H = (int)a.heads;
   p.ldq = (int)a.ldq; p.ldk = (int)a.ldk; p.ldv = (int)a.ldv; p.ldo = (int)a.ldo;
   p.Sq = (int)a.Sq; p.Sk = (int)a.Sk;
   p.D = (int)a.D;
   p.scale_log2e = scale * 1.4426950408889634f;
-  p.QB = (int)((a.Sq + 255) / 256);
+  p.QB = (int)((a.Sq + rows - 1) / rows);
   p.full_items = sp.full;
   p.parts = sp.parts;
   p.ws = ws;
+}
+
+int launch_attention(const AttnShape& a, float scale, sf_dtype dt, const AttnSplit& sp, float* ws, hipStream_t st) {
+  AttnParams p;
+  attn_fill_params(a, scale, sp, ws, 256, p);
   // One workgroup per whole item, then one per split part.
   const int64_t split_items = sp.items - sp.full;
   const int64_t wgs = sp.full + (sp.parts > 0 ? split_items * sp.parts : 0);

@@ -120,6 +120,21 @@ struct AttnSplit {
 };
 constexpr size_t kAttnPartBytes = 73728;
 AttnSplit attn_split_plan(const AttnShape& a, int cus);
+// The split of `items` work items over the keys (part_bytes of partials a part).
+AttnSplit attn_split_items(int64_t items, int64_t Sk, size_t part_bytes, int cus);
+struct AttnParams;
+void attn_fill_params(const AttnShape& a, float scale, const AttnSplit& sp, float* ws, int rows, AttnParams& p);
+// Head sizes up to 128 and additive masks (attention_wide.hpp); work items
+// are blocks of 128 query rows.
+struct AttnMask {
+  const void* ptr;  // NULL: none
+  sf_dtype dt;      // F32 or the operands' dtype
+  int64_t sB, sH, sR;  // batch, head and row strides, elements (0 broadcasts)
+};
+size_t attn_wide_part_bytes(int64_t D);
+AttnSplit attn_wide_split_plan(const AttnShape& a, int cus);
+int launch_attention_wide(const AttnShape& a, const AttnMask& m, float scale, sf_dtype dt, const AttnSplit& sp,
+                          float* ws, hipStream_t st);
 int launch_attention(const AttnShape& a, float scale, sf_dtype dt, const AttnSplit& sp, float* ws, hipStream_t st);
 // Layer norm (rms = false: centred, gamma and beta, optional per-group
 // modulation y = h (1 + scale) + shift) or RMS norm (rms = true: gamma

@@ -62,11 +62,11 @@ def dropout(input: Tensor, p: float = 0.5, training: bool = True) -> Tensor:
 def scaled_dot_product_attention(q: Tensor, k: Tensor, v: Tensor, attn_mask=None,
                                  dropout_p: float = 0.0, scale: float | None = None) -> Tensor:
     """softmax(scale * q k^T + attn_mask) v, scale defaulting to 1/sqrt(head
-    size).  16-bit inputs with a head size that is a multiple of 8 up to 64
-    and no mask run as one fused launch (sf_attention: the scores never
-    reach memory); other inputs take three launches: a strided-batched QK^T
-    with the scale in its epilogue, a row softmax with the additive mask
-    folded in, and a strided-batched PV.  The reference's GPU path
+    size).  16-bit inputs with a head size that is a multiple of 8 up to 128
+    run as one fused launch, with or without a mask (sf_attention_masked: the
+    scores never reach memory); other inputs take three launches: a
+    strided-batched QK^T with the scale in its epilogue, a row softmax with
+    the additive mask folded in, and a strided-batched PV.  The reference's GPU path
     (nn/functional.py:310-321) runs a Python loop of per-head SGEMMs, a
     scale pass, the softmax and a batched SGEMM, and sends a masked call to
     its host branch (:339-341: scores += mask, NumPy broadcasting); here

@@ -1,0 +1,167 @@
+"""Fused attention with head sizes up to 128 and additive masks
+(attention_wide.hpp) on the GPU against fp64: ragged query and key counts,
+every mask broadcast and type, rows that meet no key, a late key, large
+finite masks, split key ranges."""
+from __future__ import annotations
+
+import ctypes
+import os
+
+import numpy as np
+import pytest
+
+from helpers import cu, down, rnd, up
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LOW = float(np.finfo(np.float32).min)
+
+
+def softmax64(s):
+    m = np.max(s, -1, keepdims=True)
+    with np.errstate(invalid="ignore"):
+        e = np.exp(s - m)
+    return e / e.sum(-1, keepdims=True)
+
+
+def exact(q, k, v, scale, mask=None):
+    """fp64, with score + mask rounded to fp32 once as the device's sum is
+    (which decides rows of large finite masks)."""
+    s = scale * np.matmul(q.astype(np.float64), np.swapaxes(k, -2, -1).astype(np.float64))
+    if mask is not None:
+        s = (s.astype(np.float32) + mask.astype(np.float32)).astype(np.float64)
+    return np.matmul(softmax64(s), v.astype(np.float64))
+
+
+def check(y, y64, vmax, dtype):
+    """P and the output are rounded once each, Q once more by the pre-scaled
+    path: exponents move by up to u * sum |q_d k_d| * scale log2 e, about
+    4 u for unit-variance heads, so |error| <= (1 + 4 + 1) u max|v| with u the
+    type's half ulp."""
+    u = {"float16": 2.0 ** -11, "bfloat16": 2.0 ** -8}[dtype]
+    assert np.array_equal(np.isnan(y), np.isnan(y64))
+    ok = ~np.isnan(y64)
+    err = np.abs(y.astype(np.float64) - y64)[ok]
+    assert err.max() <= 6 * u * vmax, err.max()
+
+
+def masks(kind, b, h, sq, sk, rng, dtype):
+    if kind == "causal":
+        return np.where(np.arange(sk)[None, :] > np.arange(sq)[:, None] + max(0, sk - sq), -np.inf, 0.0)
+    if kind == "pad":  # [B, 1, 1, Sk]: the second half, and all but one key of the last sample
+        m = np.zeros((b, 1, 1, sk))
+        m[0, ..., sk // 2:] = -np.inf
+        m[-1, ..., :] = -np.inf
+        m[-1, ..., sk - 1] = 0.0
+        return m
+    if kind == "left-low":  # only the last keys count; the earlier ones hold the lowest value or -1e9
+        m = np.zeros((b, 1, 1, sk))
+        m[0, ..., : sk - 3] = LOW
+        m[-1, ..., : sk - 3] = -1e9
+        return m
+    if kind == "rows":  # whole rows at -inf (NaN), the lowest value, -1e9, and a mixture
+        m = np.zeros((h, sq, sk))
+        m[:, 0] = -np.inf
+        m[:, sq // 2] = LOW
+        m[:, sq // 3] = -1e9
+        m[:, sq - 1] = -np.inf
+        m[:, sq - 1, sk // 2:] = LOW
+        return m
+    return rnd(rng, (b, h, sq, sk), 3.0, dtype)  # "bias"
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("d", [72, 96, 104, 128])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 127, 65), (3, 129, 64), (1, 300, 1000)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_wide_heads(dtype, d, shape):
+    bh, sq, sk = shape
+    rng = np.random.default_rng(d + sq + sk)
+    q, k, v = (rnd(rng, (bh, s, d), 1.0, dtype) for s in (sq, sk, sk))
+    y = down(cu().dev_scaled_dot_product_attention(up(q, dtype), up(k, dtype), up(v, dtype)))
+    check(y, exact(q, k, v, d ** -0.5), np.abs(v).max(), dtype)
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("d,scale", [(40, None), (64, None), (64, 1.0), (80, None), (128, None)])
+@pytest.mark.parametrize("kind,mdtype", [("causal", "float32"), ("pad", "float32"), ("left-low", "float32"),
+                                         ("rows", "float32"), ("bias", "float32"), ("bias", None)])
+def test_masks(dtype, d, scale, kind, mdtype):
+    """Sk = 203 (a partial last block, mask rows at no 16-byte boundary) and
+    two batch entries of three heads; scale 1 takes the FMA path."""
+    b, h, sq, sk = 2, 3, 133, 203
+    rng = np.random.default_rng(d + len(kind))
+    q, k, v = (rnd(rng, (b, h, s, d), 0.5 if scale else 1.0, dtype) for s in (sq, sk, sk))
+    m = masks(kind, b, h, sq, sk, rng, dtype).astype(np.float32)
+    gm = up(m, mdtype or dtype)
+    y = down(cu().dev_scaled_dot_product_attention(up(q, dtype), up(k, dtype), up(v, dtype), scale, gm))
+    check(y, exact(q, k, v, scale or d ** -0.5, m), np.abs(v).max(), dtype)
+
+
+@pytest.mark.parametrize("kind", ["none", "causal", "left-low", "rows"])
+@pytest.mark.parametrize("d", [64, 128])
+def test_split_key_ranges(kind, d):
+    """Every item in three key ranges (test hook): parts in which a row meets
+    no key weigh nothing, rows without any key are finished by the merge."""
+    b, h, sq, sk = 2, 2, 130, 700
+    rng = np.random.default_rng(d)
+    q, k, v = (rnd(rng, (b, h, s, d), 1.0, "bfloat16") for s in (sq, sk, sk))
+    m = None if kind == "none" else masks(kind, b, h, sq, sk, rng, "bfloat16").astype(np.float32)
+    g = cu()
+    g._set_test_hooks(attn_parts=3)
+    try:
+        y = down(g.dev_scaled_dot_product_attention(up(q, "bfloat16"), up(k, "bfloat16"), up(v, "bfloat16"), None,
+                                                    None if m is None else up(m, "float32")))
+    finally:
+        g._set_test_hooks()
+    check(y, exact(q, k, v, d ** -0.5, m), np.abs(v).max(), "bfloat16")
+
+
+def test_nan_and_inf_scores_reach_their_rows():
+    """A NaN in one query row and an infinite key: the rows that a plain
+    softmax makes NaN are NaN, and no other."""
+    rng = np.random.default_rng(3)
+    q, k, v = (rnd(rng, (1, s, 128), 1.0, "bfloat16") for s in (100, 90, 90))
+    q[0, 7, 3] = np.nan
+    k[0, 50, 5] = np.inf
+    m = np.zeros((100, 90), np.float32)
+    m[20:, 50] = -np.inf
+    y = down(cu().dev_scaled_dot_product_attention(up(q, "bfloat16"), up(k, "bfloat16"), up(v, "bfloat16"), None,
+                                                   up(m, "float32")))
+    with np.errstate(invalid="ignore"):
+        s = 128 ** -0.5 * np.matmul(q.astype(np.float64), np.swapaxes(k, -2, -1).astype(np.float64)) + m
+        y64 = np.matmul(softmax64(s), v.astype(np.float64))
+    assert np.array_equal(np.isnan(y), np.isnan(y64))
+
+
+def test_packed_heads_of_80_and_columns_past_d():
+    """Heads of 80 read in place from a packed projection (the 96-wide tile
+    must not take its neighbour's columns), written side by side."""
+    b, n, h, d = 2, 150, 3, 80
+    rng = np.random.default_rng(8)
+    qkv = rnd(rng, (b, n, 3 * h * d), 1.0, "float16")
+    y = down(cu().dev_attention_packed(up(qkv, "float16"), h))
+    q, k, v = (x.reshape(b, n, h, d).transpose(0, 2, 1, 3) for x in np.split(qkv, 3, -1))
+    check(y, exact(q, k, v, d ** -0.5).transpose(0, 2, 1, 3).reshape(b, n, h * d), np.abs(v).max(), "float16")
+
+
+def test_abi_rules():
+    """sf_attention keeps refusing head sizes above 64; the masked entry
+    refuses what neither takes."""
+    lib = ctypes.CDLL(os.path.join(ROOT, "scaffolding_amd", "libsfgemm.so"))
+    I64, P, F = ctypes.c_int64, ctypes.c_void_p, ctypes.c_float
+    x = up(np.zeros((64, 136), np.float32), "bfloat16")
+
+    def masked(d, mdt, row, dt=2):
+        p = P(x.data_ptr)
+        s = [I64(136), I64(0), I64(0)]
+        o = [I64(136), I64(64 * 136), I64(64 * 136)]
+        return lib.sf_attention_masked(p, *s, p, *s, p, *s, p, *o, I64(1), I64(1), I64(8), I64(8), I64(d), F(0.1), dt,
+                                       p, mdt, I64(0), I64(0), I64(row), None)
+
+    assert masked(136, 2, 0) == -3 and masked(12, 2, 0) == -3 and masked(64, 2, 0, dt=0) == -3
+    assert masked(64, 1, 0) == -3 and masked(64, 7, 0) == -2 and masked(64, 2, -1) == -2
+    p = P(x.data_ptr)
+    assert lib.sf_attention(p, I64(80), I64(0), p, I64(80), I64(0), p, I64(80), I64(0), p, I64(80), I64(0), I64(1),
+                            I64(8), I64(8), I64(80), F(0.1), 2, None) == -3
