@@ -67,4 +67,37 @@ template <typename T> struct Chunk8 {  // BF16 / F16
   }
 };
 
+// 16-byte chunks at element alignment (one dwordx4 access each: global
+// accesses need no more on this target).
+struct __attribute__((packed, aligned(4))) F4u {
+  f32x4 v;
+};
+struct __attribute__((packed, aligned(2))) H8u {
+  u32x4 v;
+};
+template <typename T>
+__device__ __forceinline__ void load8u(const void* base, int64_t i, float v[8]) {
+  if constexpr (std::is_same<T, float>::value) {
+    const F4u* p = reinterpret_cast<const F4u*>(static_cast<const float*>(base) + i);
+    const f32x4 a = p[0].v, b = p[1].v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { v[e] = a[e]; v[e + 4] = b[e]; }
+  } else {
+    const u32x4 w = reinterpret_cast<const H8u*>(static_cast<const uint16_t*>(base) + i)->v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = Elem<T>::to_f32(static_cast<uint16_t>(w[e >> 1] >> ((e & 1) * 16)));
+  }
+}
+template <typename T>
+__device__ __forceinline__ void store8u(void* base, int64_t i, const float v[8]) {
+  if constexpr (std::is_same<T, float>::value) {
+    F4u* p = reinterpret_cast<F4u*>(static_cast<float*>(base) + i);
+    p[0].v = f32x4{v[0], v[1], v[2], v[3]};
+    p[1].v = f32x4{v[4], v[5], v[6], v[7]};
+  } else {
+    reinterpret_cast<H8u*>(static_cast<uint16_t*>(base) + i)->v =
+        u32x4{pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3]), pack2<T>(v[4], v[5]), pack2<T>(v[6], v[7])};
+  }
+}
+
 }  // namespace sf
