@@ -851,6 +851,19 @@ static int attn_prepare(const char* name, const void* Q, int64_t ldq, int64_t st
   return SF_OK;
 }
 
+static int attn_wide_run(const AttnShape& a, const AttnMask& m, float scale, sf_dtype dtype, int cus, hipStream_t st) {
+  const AttnSplit sp = attn_wide_split_plan(a, cus);
+  if (sp.parts == 0) return launch_attention_wide(a, m, scale, dtype, sp, nullptr, st);
+  float* ws = nullptr;
+  int* cnt = nullptr;
+  int rc = split_workspace_acquire((size_t)(sp.items - sp.full) * (size_t)sp.parts * attn_wide_part_bytes(a.D), 0, st,
+                                   &ws, &cnt);
+  if (rc != SF_OK) return rc;
+  rc = launch_attention_wide(a, m, scale, dtype, sp, ws, st);
+  const int rc2 = split_workspace_release(st);
+  return rc != SF_OK ? rc : rc2;
+}
+
 int sf_attention_heads(const void* Q, int64_t ldq, int64_t strideQ, int64_t headQ, const void* K, int64_t ldk,
                        int64_t strideK, int64_t headK, const void* V, int64_t ldv, int64_t strideV, int64_t headV,
                        void* O, int64_t ldo, int64_t strideO, int64_t headO, int64_t batch, int64_t heads,
@@ -861,7 +874,17 @@ int sf_attention_heads(const void* Q, int64_t ldq, int64_t strideQ, int64_t head
                         ldo, strideO, headO, batch, heads, Sq, Sk, D, 64, scale, dtype, a, &noop);
   if (rc != SF_OK || noop) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const AttnSplit sp = attn_split_plan(a, cu_count_current());
+  const int cus = cu_count_current();
+  // At most one 256-row item per CU: the 128-row items of the wide kernel
+  // fill the GPU better (30 heads, 1350 tokens 37.2 -> 30.4 us; 226 keys
+  // 16.0 -> 10.5 us; 64 heads, 1024 tokens 37.2 -> 25.5 us; 12 heads, 4096
+  // tokens 76 -> 71 us).  With more items its second read of K and V costs
+  // more (48 heads, 2048 tokens 62.7 against 68.5 us), and so it does where
+  // few items are split over many keys (8 heads, 2048 x 8192 50.2 against
+  // 52.2 us).
+  if (batch * heads * cdiv(Sq, 256) <= cus && !(Sk > 4096 && Sq >= 256))
+    return attn_wide_run(a, AttnMask{nullptr, dtype, 0, 0, 0}, scale, dtype, cus, st);
+  const AttnSplit sp = attn_split_plan(a, cus);
   if (sp.parts == 0) return launch_attention(a, scale, dtype, sp, nullptr, st);
   float* ws = nullptr;
   int* cnt = nullptr;
@@ -895,17 +918,7 @@ int sf_attention_masked(const void* Q, int64_t ldq, int64_t strideQ, int64_t hea
       return fail(SF_ERR_INVALID_ARG, "sf_attention_masked: negative mask stride");
   }
   if (noop) return SF_OK;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const AttnSplit sp = attn_wide_split_plan(a, cu_count_current());
-  if (sp.parts == 0) return launch_attention_wide(a, m, scale, dtype, sp, nullptr, st);
-  float* ws = nullptr;
-  int* cnt = nullptr;
-  rc = split_workspace_acquire((size_t)(sp.items - sp.full) * (size_t)sp.parts * attn_wide_part_bytes(D), 0, st, &ws,
-                               &cnt);
-  if (rc != SF_OK) return rc;
-  rc = launch_attention_wide(a, m, scale, dtype, sp, ws, st);
-  const int rc2 = split_workspace_release(st);
-  return rc != SF_OK ? rc : rc2;
+  return attn_wide_run(a, m, scale, dtype, cu_count_current(), static_cast<hipStream_t>(stream));
 }
 
 int sf_attention(const void* Q, int64_t ldq, int64_t strideQ, const void* K, int64_t ldk, int64_t strideK,

@@ -110,6 +110,16 @@ __device__ __forceinline__ AttnItem attn_item(const AttnParams& p, int64_t it, i
   return w;
 }
 
+// The place of this workgroup among its launch's: each XCD takes a contiguous
+// range of the whole items and one of the split parts, so the query blocks
+// of one head share its L2 copy of K and V (60 heads, 4096 tokens 249 -> 236.5 us).
+__device__ __forceinline__ int attn_slot(const AttnParams& p) {
+  const int64_t left = p.full_items - p.item0;
+  const int bid = (int)blockIdx.x, n = (int)gridDim.x;
+  const int nfull = left <= 0 ? 0 : (left < (int64_t)n ? (int)left : n);
+  return bid < nfull ? xcd_remap(bid, nfull) : nfull + xcd_remap(bid - nfull, n - nfull);
+}
+
 // Normalised output rows of one wave: row block mb's 16 rows from the
 // accumulator layout (lane l: query l % 16, d = 16 db + 4 (l / 16) + 0..3),
 // columns at or past D not stored.
@@ -153,7 +163,7 @@ __global__ __launch_bounds__(256, 2) void attn64_kernel(AttnParams p) {
   // buffer bound) and its scores there are masked to -inf.
   const int NB = (Sk + KB - 1) / KB;
   const int k_tail = Sk - (NB - 1) * KB;  // valid keys of the last block, 1..64
-  const AttnItem wi = attn_item(p, p.item0 + blockIdx.x, NB);
+  const AttnItem wi = attn_item(p, p.item0 + attn_slot(p), NB);
   const int64_t b = wi.b, h = wi.h;
   const int q0 = wi.qb * 256 + wave * 64;
   const int kb0 = wi.kb0, kb1 = wi.kb1;

@@ -34,6 +34,7 @@ template <typename T>
 static int launch_wide_t(int dw, int mk, const AttnWideParams& wp, bool pre, int64_t wgs, int64_t split_items,
                          hipStream_t st) {
   switch (dw * 4 + mk) {
+    case 64 * 4 + 0: return launch_wide<T, 64, 0>(wp, pre, wgs, split_items, st);
     case 64 * 4 + 1: return launch_wide<T, 64, 1>(wp, pre, wgs, split_items, st);
     case 64 * 4 + 2: return launch_wide<T, 64, 2>(wp, pre, wgs, split_items, st);
     case 96 * 4 + 0: return launch_wide<T, 96, 0>(wp, pre, wgs, split_items, st);

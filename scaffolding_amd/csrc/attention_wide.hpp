@@ -27,8 +27,9 @@
 // the scores in memory):
 //   2 x 16 heads, 2048 x 2048, D 128          278 -> 64 us   (1080 TFLOP/s)
 //   2 x 24 heads, 8192 x 8192, D 128             1.38 ms     (1200 TFLOP/s)
-//   1 x 30 heads, 7239 x 7239, D 72        7.6 ms -> 0.73 ms
-//   4 x 16 heads, 1024 x 1024, D 64, causal mask 127 -> 41 us
+//   1 x 30 heads, 7239 x 7239, D 72        7.6 ms -> 0.56 ms
+//   4 x 16 heads, 1024 x 1024, D 64, causal mask 127 -> 40 us
+//   1 x 30 heads, 1350 x 1350, D 64           37.2 -> 30.4 us (attn64_kernel)
 #pragma once
 
 #include "attention.hpp"
@@ -192,13 +193,7 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
   const int Sq = p.Sq, Sk = p.Sk;
   const int NB = (Sk + KB - 1) / KB;
   const int k_tail = Sk - (NB - 1) * KB;
-  // Each XCD takes a contiguous range of the whole items and one of the split
-  // parts, so the query blocks of one head share its L2 copy of K and V.
-  const int64_t left = p.full_items - p.item0;
-  const int nfull = left <= 0 ? 0 : (left < (int64_t)gridDim.x ? (int)left : (int)gridDim.x);
-  const int bid = (int)blockIdx.x;
-  const int slot = bid < nfull ? xcd_remap(bid, nfull) : nfull + xcd_remap(bid - nfull, (int)gridDim.x - nfull);
-  const AttnItem wi = attn_item(p, p.item0 + slot, NB);
+  const AttnItem wi = attn_item(p, p.item0 + attn_slot(p), NB);
   const int64_t b = wi.b, h = wi.h;
   const int q0 = wi.qb * C::ROWS + wave * (MB * 16);
   const int kb0 = wi.kb0, kb1 = wi.kb1;
@@ -339,9 +334,8 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
       });
     };
     // REF: the exponents, against the row references (with PRE the mask and
-    // the reference are the score MFMAs' C operand; the mask is rounded into
-    // the exponent domain before the reference is added, so equal mask
-    // values stay equal whatever the reference).  Otherwise scores + mask,
+    // the reference are the score MFMAs' C operand: one FMA, whose rounding
+    // is that of the reference, at most 2^8).  Otherwise scores + mask,
     // rounded as one fp32 sum, without a reference.
     auto scores = [&](auto ref_c) {
       constexpr bool REF = decltype(ref_c)::value;
@@ -364,11 +358,7 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
             c = nq[mb];
             if constexpr (MK != 0) {
 #pragma unroll
-              for (int q = 0; q < 4; ++q) {
-#pragma clang fp contract(off)
-                const float m2 = mk[mb][NBK][q] * LOG2E;
-                c[q] = m2 + nq[mb][q];
-              }
+              for (int q = 0; q < 4; ++q) c[q] = __builtin_fmaf(mk[mb][NBK][q], LOG2E, nq[mb][q]);
             }
           }
           s[mb][NBK] = Mfma16<T>::run(kf[0], qf[mb][0], c);
@@ -393,8 +383,11 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
 #pragma clang fp contract(off)
               float add = REF ? nq[mb][q] : 0.f;
               if constexpr (MK != 0) {
-                const float m2 = mk[mb][nb][q] * LOG2E;
-                add = m2 + add;
+                if constexpr (REF) {
+                  add = __builtin_fmaf(mk[mb][nb][q], LOG2E, add);
+                } else {
+                  add = mk[mb][nb][q] * LOG2E;
+                }
               }
               s[mb][nb][q] = PRE ? s[mb][nb][q] + add : __builtin_fmaf(s[mb][nb][q], p.scale_log2e, add);
             }
