@@ -150,7 +150,8 @@ static int cu_count_current() {
 // split ov0 + ov1 * parts (partials and their sum).  Fitted to sweeps on one
 // MI355X of 133 aligned problems (M 24-6400, N 640-11008, K 104-7680, NT, NN
 // and TN): the plan the estimate picks is on average 1.6 % slower than the
-// fastest one measured, at worst 16 %; 29 unaligned ones: 7 %.
+// fastest one measured, at worst 16 %; 29 unaligned ones: 2.7 %, at worst
+// 17 %.
 struct MidCost {
   int cfg, bm, bn, occ;
   float tau[4];
@@ -162,14 +163,14 @@ static const MidCost kMidAligned[] = {
     {TILE_MID_32, 32, 64, 3, {0.185f, 0.25f, 0.40f}, 1.5f, 1.2f, 0.2f},
 };
 // Register-staged loads of k-contiguous rows, and of operands with k-rows
-// (two transposing reads a fragment, unaligned k-rows): about 1.8x the time.
+// (two transposing reads a fragment, unaligned k-rows).
 static const MidCost kMidRagged[] = {
-    {TILE_RAG_128, 128, 128, 2, {1.1f, 1.5f}, 3.0f, 6.0f, 1.0f},
-    {TILE_RAG_64, 64, 64, 4, {0.42f, 0.80f, 1.15f, 1.75f}, 2.0f, 2.0f, 0.3f},
+    {TILE_RAG_128, 128, 128, 2, {0.9f, 1.5f}, 3.0f, 4.0f, 1.2f},
+    {TILE_RAG_64, 64, 64, 4, {0.45f, 0.85f, 1.1f, 1.75f}, 2.0f, 2.0f, 0.3f},
 };
 static const MidCost kMidRaggedMn[] = {
-    {TILE_RAG_128, 128, 128, 2, {1.4f, 2.7f}, 3.0f, 6.0f, 1.0f},
-    {TILE_RAG_64, 64, 64, 4, {0.75f, 1.2f, 1.75f, 2.3f}, 2.0f, 2.0f, 0.3f},
+    {TILE_RAG_128, 128, 128, 2, {1.2f, 1.8f}, 3.0f, 4.0f, 1.2f},
+    {TILE_RAG_64, 64, 64, 4, {0.9f, 1.6f, 1.9f, 2.4f}, 2.0f, 2.0f, 0.3f},
 };
 constexpr int kMaxSplitMid = 8;
 constexpr float kMidFixed = 5.0f;  // launch, first loads, epilogue

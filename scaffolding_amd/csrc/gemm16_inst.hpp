@@ -63,7 +63,7 @@ static int launch16_t(int cfg, const GemmParams& p, unsigned gx, unsigned gy, hi
       }
       return fail(SF_ERR_UNSUPPORTED, "the 32x64 tile needs K-contiguous A and B");
     case TILE_RAG_128:
-      hipLaunchKernelGGL((gemm16mid_kernel<TIn, TOut, 128, 128, 2, 2, 2, AKM, KM, false, 2>), g, dim3(256), 0, st, p);
+      hipLaunchKernelGGL((gemm16mid_kernel<TIn, TOut, 128, 128, 2, 4, 2, AKM, KM, false, 4>), g, dim3(512), 0, st, p);
       break;
     case TILE_RAG_64:
       hipLaunchKernelGGL((gemm16mid_kernel<TIn, TOut, 64, 64, 2, 2, 2, AKM, KM, false, 4>), g, dim3(256), 0, st, p);

@@ -38,7 +38,9 @@
 //  2048 x 1920 x 7680 NN    82.8 -> 64.6 us   128 x 128, 2 parts
 //  1920 x 1920 x 2048 TN    50.2 -> 26.2 us   128 x 128
 //   777 x 1283 x 1001 NT    47.2 -> 14.7 us   64 x 64, unaligned
-//   515 x 4097 x 2001 TN   217   -> 43.9 us   128 x 128, 3 parts, unaligned
+//   515 x 4097 x 2001 TN   217   -> 33.6 us   128 x 128, 3 parts, unaligned
+// (Two, three or four unaligned slices held in registers instead of one:
+// within 3 %; the unaligned accesses themselves are the limit.)
 #pragma once
 
 #include "gemm16nt_pp.hpp"
