@@ -160,6 +160,13 @@ _F16 = np.dtype(np.float16)
 
 
 cdef sf_dtype _sf_dtype(object dt) except *:
+    # the dtype objects themselves first: comparing dtypes costs a few 100 ns
+    if dt is _F32:
+        return SF_F32
+    if dt is BFLOAT16:
+        return SF_BF16
+    if dt is _F16:
+        return SF_F16
     d = np.dtype(dt) if not isinstance(dt, np.dtype) else dt
     if d == _F32:
         return SF_F32
@@ -171,18 +178,22 @@ cdef sf_dtype _sf_dtype(object dt) except *:
 
 
 cdef size_t _itemsize(object dt) except 0:
+    if dt is _F32:
+        return 4
+    if dt is BFLOAT16 or dt is _F16:
+        return 2
     return (<object>np.dtype(dt)).itemsize
 
 
 def resolve_dtype(dt):
     """Maps 'bfloat16' / 'float16' / 'float32' / numpy dtypes to the device
     storage dtype used in GpuTensor.dtype."""
+    if isinstance(dt, np.dtype):
+        return dt
     if isinstance(dt, str):
         if dt in ('bfloat16', 'bf16'):
             return BFLOAT16
         return np.dtype(dt)
-    if isinstance(dt, np.dtype):
-        return dt
     return np.dtype(dt)
 
 
@@ -285,13 +296,17 @@ def set_cache_limit(size_t nbytes):
 #  GpuTensor (reference _cuda_ops.pyx:807-819)
 # ================================================================
 
-class GpuTensor:
+cdef class GpuTensor:
     """GPU-resident, C-contiguous tensor: a CudaBuffer plus shape and dtype."""
-    __slots__ = ('buffer', 'shape', 'dtype', 'numel', 'device_id')
+    cdef public object buffer
+    cdef public object shape
+    cdef public object dtype
+    cdef public object numel
+    cdef public object device_id
 
     def __init__(self, buffer, tuple shape, dtype, int device_id=-1):
         self.buffer = buffer
-        self.shape = tuple(int(s) for s in shape)
+        self.shape = tuple([int(s) for s in shape])
         self.dtype = resolve_dtype(dtype)
         self.device_id = device_id if device_id >= 0 else (<CudaBuffer>buffer).device_id
         cdef int64_t n = 1
@@ -317,18 +332,27 @@ cdef inline void* _ptr(gt) except? NULL:
 
 
 cdef object _alloc_like(tuple shape, dtype, int device_id):
+    """New device tensor; shape holds Python ints and dtype is a storage
+    dtype (both as a GpuTensor's own), so neither is normalised again."""
     cdef int64_t n = 1
     for s in shape:
         n *= s
     cdef size_t nbytes = <size_t>n * _itemsize(dtype)
-    return GpuTensor(_make_buffer(nbytes, device_id), shape, dtype, device_id)
+    cdef CudaBuffer buf = _make_buffer(nbytes, device_id)
+    cdef GpuTensor out = GpuTensor.__new__(GpuTensor)
+    out.buffer = buf
+    out.shape = shape
+    out.dtype = dtype
+    out.numel = n
+    out.device_id = device_id if device_id >= 0 else buf.device_id
+    return out
 
 
 def empty(tuple shape, dtype=np.float32, int device_id=-1):
     """Uninitialised device tensor."""
     if device_id < 0:
         device_id = _current_device()
-    return _alloc_like(shape, resolve_dtype(dtype), device_id)
+    return _alloc_like(tuple([int(s) for s in shape]), resolve_dtype(dtype), device_id)
 
 
 def zeros(tuple shape, dtype=np.float32, int device_id=-1):
@@ -593,6 +617,8 @@ cdef class CudaEvent:
 # ================================================================
 
 cdef object _same_dtype(a, b, str name):
+    if a.dtype is b.dtype:
+        return a.dtype
     if a.dtype != b.dtype:
         raise TypeError("%s: operand dtypes differ (%s vs %s)" % (name, a.dtype, b.dtype))
     return a.dtype

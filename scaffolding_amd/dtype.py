@@ -13,6 +13,10 @@ import numpy as np
 from . import _cuda_ops as _cuops
 
 
+_F32 = np.dtype(np.float32)
+_F16 = np.dtype(np.float16)
+
+
 class dtype(enum.Enum):
     float16 = "float16"
     float32 = "float32"
@@ -30,6 +34,14 @@ class dtype(enum.Enum):
 
     @staticmethod
     def from_any(d) -> "dtype":
+        # The storage dtypes' own objects first: this runs once per operator
+        # result, and comparing NumPy dtypes costs a few 100 ns.
+        if d is _F32:
+            return dtype.float32
+        if d is _cuops.BFLOAT16:
+            return dtype.bfloat16
+        if d is _F16:
+            return dtype.float16
         if isinstance(d, dtype):
             return d
         if isinstance(d, str):

@@ -53,7 +53,10 @@ class Tensor:
         t = cls.__new__(cls)
         t._data = None
         t._gpu = gt
-        t._device = _device_t(device) if device is not None else _device_t("cuda:%d" % gt.device_id)
+        if isinstance(device, _device_t):
+            t._device = device  # immutable: shared
+        else:
+            t._device = _device_t(device) if device is not None else _device_t("cuda:%d" % gt.device_id)
         t._dtype = _dtype_t.from_any(gt.dtype)
         t._requires_grad = requires_grad
         return t
