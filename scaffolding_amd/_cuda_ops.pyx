@@ -1046,7 +1046,7 @@ cdef object _mha_strided(q, int64_t q_off, int64_t ldq, k, int64_t k_off, int64_
     cdef char* pv = <char*>_ptr(v) + v_off * es
     cdef char* po = <char*>_ptr(out)
     cdef int ret = SF_ERR_UNSUPPORTED
-    if sdt != SF_F32 and 8 <= D <= 128 and D % 8 == 0 and scale > 0:
+    if sdt != SF_F32 and 8 <= D <= (128 if Sk > 0 else 64) and D % 8 == 0 and scale > 0:
         with nogil:
             ret = sf_attention_masked(pq, ldq, Nq * ldq, D, pk, ldk, Sk * ldk, D, pv, ldv, Sk * ldv, D,
                                       po, C, Nq * C, D, B, H, Nq, Sk, D, scale, sdt, NULL, sdt, 0, 0, 0, NULL)
@@ -1341,6 +1341,10 @@ def dev_scaled_dot_product_attention(q, k, v, scale=None, attn_mask=None, float 
         raise ValueError("dev_scaled_dot_product_attention: dropout_p must be in [0, 1), got %r" % dropout_p)
     if dropout_p > 0.0 or q.dtype == np.float32 or d < 8 or d > 128 or d % 8 != 0 or not (0.0 < s < 3.0e38):
         return dev_sdpa_unfused(q, k, v, scale, attn_mask, dropout_p, seed, offset)
+    # Nothing to launch on: only the three-launch path takes empty batches
+    # with a mask (whose groups may be empty too) and rows without a key.
+    if (attn_mask is not None or d > 64) and (batch == 0 or sq == 0 or sk == 0):
+        return dev_sdpa_unfused(q, k, v, scale, attn_mask)
     # The mask's broadcast over the leading dims, as an outer and an inner
     # group of them (batch entries and heads of the fused kernel).
     cdef void* pm = NULL

@@ -146,6 +146,21 @@ def test_packed_heads_of_80_and_columns_past_d():
     check(y, exact(q, k, v, d ** -0.5).transpose(0, 2, 1, 3).reshape(b, n, h * d), np.abs(v).max(), "float16")
 
 
+@pytest.mark.parametrize("shape", [(0, 4, 16, 16), (2, 0, 16, 16), (2, 3, 0, 16), (2, 3, 16, 0)],
+                         ids=["batch", "heads", "queries", "keys"])
+@pytest.mark.parametrize("d,masked", [(64, True), (128, False), (128, True)])
+def test_empty_operands(shape, d, masked):
+    """Empty batches, and rows without a key, give what the three launches
+    give: an empty result, zeros."""
+    b, h, sq, sk = shape
+    g = cu()
+    q, k, v = (g.zeros((b, h, s, d), g.BFLOAT16) for s in (sq, sk, sk))
+    for m in [(sq, sk), (b, 1, sq, sk)] if masked else [None]:
+        gm = None if m is None else g.zeros(m, np.float32)
+        y = g.dev_scaled_dot_product_attention(q, k, v, None, gm)
+        assert y.shape == (b, h, sq, d) and not down(y).any()
+
+
 def test_abi_rules():
     """sf_attention keeps refusing head sizes above 64; the masked entry
     refuses what neither takes."""
