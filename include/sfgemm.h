@@ -131,7 +131,7 @@ int sf_set_test_hooks(int xcd_shift, int split_spins, int attn_parts);
  * The call is asynchronous on `stream`.  Some plans split tiles along k and
  * pass fp32 partials through a per-device workspace, allocated on first use
  * (see sf_gemm_noalloc).  On a stream that is being captured, mid-size 16-bit
- * problems (fewer than one 256 x 256 tile per CU, or unaligned operands) run
+ * problems (fewer than one 256 x 256 tile per CU) and unaligned operands run
  * without that split, so capturing them allocates nothing. */
 int sf_gemm(int transA, int transB,
             int64_t M, int64_t N, int64_t K, int64_t batch,

@@ -64,6 +64,8 @@ const char* tile_name(int cfg) {
     case TILE_MID_32: return "gemm tile 32x64";
     case TILE_RAG_128: return "gemm tile generic 128x128";
     case TILE_RAG_64: return "gemm tile generic 64x64";
+    case TILE32_RAG: return "gemm tile generic 64x64 lds-dma k-groups";
+    case TILE32_RAG_SPLIT: return "gemm tile generic 64x64 lds-dma";
   }
   return "gemm";
 }
@@ -284,10 +286,25 @@ static int choose_tile16(int64_t M, int64_t N, int64_t K, int64_t batch, bool ve
 // register-staged; 4096^3 NN 85% of the fp32 MFMA peak against 77%.
 static int choose_tile32(int64_t M, int64_t N, int64_t K, int64_t batch, bool vec, bool a_kmajor, bool dma_ok,
                          int cus) {
-  if (!vec) return TILE_GENERIC;
+  // Unaligned operands (TILE_GENERIC loads element by element through
+  // registers: 2 GiB and more): 777 x 1283 x 1001 NT 76.9 -> 48 us, 4001 x
+  // 2003 x 1001 NT 298 -> 178 us, 33 x 1025 x 4097 NT 136 -> 25.2 us in 8
+  // parts, TN 1001 x 1003 x 2001 86.6 -> 44.5 us.
+  if (!vec) return dma_ok ? TILE32_RAG : TILE_GENERIC;
   if (a_kmajor && 4 * cdiv(M, 64) * cdiv(N, 64) * batch <= cus && K <= 2048)
     return 2 * cdiv(M, 16) * cdiv(N, 16) * batch <= cus ? TILE32_SMALL1 : TILE32_SMALL2;
-  if (dma_ok) return (K / 32) % 2 == 0 ? TILE32_DMA : TILE32_DMA_SPLIT;
+  if (dma_ok && a_kmajor && K % 32 == 0) return (K / 32) % 2 == 0 ? TILE32_DMA : TILE32_DMA_SPLIT;
+  // An M-contiguous A, or a K that is no multiple of 32: the same kernel from
+  // one 64 x 64 tile per CU on, until the 128 x 128 register-staged tiles
+  // fill the CUs (TN 1024 x 1024 x 2048 61.8 -> 39.1 us, 1920 x 1920 x 2048
+  // 174 -> 133 us; NN 1000^3 32.1 -> 22.3 us; 4096 x 1024 x 4096 the same),
+  // and where few TN tiles are split (512 x 512 x 4096 63.8 -> 43.8 us).  In
+  // between the split 128 x 128 tiles have fewer partials to sum (TN 768 x
+  // 768 x 2048 49.8 us against 71.1 in 8 parts of 64 x 64).
+  const int64_t t64 = cdiv(M, 64) * cdiv(N, 64) * batch;
+  if (dma_ok && K >= 128 && cdiv(M, 128) * cdiv(N, 128) * batch < cus &&
+      (t64 >= cus || (!a_kmajor && 4 * t64 <= cus)))
+    return TILE32_DMA;
   if (cdiv(M, 128) * cdiv(N, 128) * batch >= cus) return TILE_128x128;
   return TILE_64x64;
 }
@@ -514,11 +531,16 @@ int gemm_prepare(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
   int bm, bn, mid_split = 0;
   if (ab_dtype == SF_F32) {
     const bool vec = al16(A) && al16(B) && (lda % 4 == 0) && (ldb % 4 == 0) &&
-                     (strideA % 4 == 0) && (strideB % 4 == 0) && (K % 4 == 0) &&
+                     (strideA % 4 == 0) && (strideB % 4 == 0) && (K % 4 == 0 || (!a_kmajor && !b_kmajor)) &&
                      (a_kmajor || M % 4 == 0) && (b_kmajor || N % 4 == 0);
-    // The LDS-DMA kernel addresses each operand with 32-bit byte offsets.
-    const bool dma_ok = a_kmajor && K % 32 == 0 && M * lda * 4 < (int64_t(1) << 31) &&
-                        (b_kmajor ? N : K) * ldb * 4 < (int64_t(1) << 31);
+    // The LDS-DMA kernel addresses each operand, and up to 64 k-rows past
+    // its end where its slices run past K, with 32-bit byte offsets.
+    const int64_t krows = K % 64 == 0 || (vec && a_kmajor && K % 32 == 0) ? K : K + 64;
+    auto fits = [&](bool kmajor, int64_t rows, int64_t ld) {
+      return (kmajor ? rows : krows) * ld * 4 < (int64_t(1) << 31);
+    };
+    auto al4 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 3) == 0; };
+    const bool dma_ok = fits(a_kmajor, M, lda) && fits(b_kmajor, N, ldb) && al4(A) && al4(B) && al4(C);
     plan.fp32 = true;
     plan.cfg = choose_tile32(M, N, K, batch, vec, a_kmajor, dma_ok, cus);
   } else {
@@ -549,19 +571,24 @@ int gemm_prepare(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
   p.wave4 = 0;
   p.xcd_shift = 0;
   p.arrive_spins = kSplitArriveSpins;
-  if (plan.fp32 && batch == 1 && K >= 128 && (plan.cfg == TILE32_DMA || plan.cfg == TILE32_DMA_SPLIT)) {
+  const bool rag32 = plan.fp32 && plan.cfg == TILE32_RAG;
+  if (plan.fp32 && batch == 1 && K >= 128 && (plan.cfg == TILE32_DMA || plan.cfg == TILE32_DMA_SPLIT || rag32)) {
     // LDS-DMA fp32 with at most CUs / 4 tiles of 64 x 64 (K > 2048, past the
     // small-block kernel): split every tile along k, at most 8 parts of at
     // least 4 slices (64 x 4096 x 4096 NT: 37.9 us in 4 parts against
     // 52 us small 16 x 32 blocks and 72 us unsplit; 200 x 300 x 4096 NN:
     // 21.5 us in 8 parts against 71.6 us unsplit).  With more tiles two
-    // k-groups beat two k-parts (768 x 768 x 1024 NN: 21.9 us against 27 us).
-    const int64_t t64 = cdiv(M, 64) * cdiv(N, 64), KT = K / 32;
-    int64_t sp = cus / (t64 > 0 ? t64 : 1);
+    // k-groups beat two k-parts (768 x 768 x 1024 NN: 21.9 us against 27 us)
+    // but for unaligned operands of long k (512 x 1001 x 8193 NT: 118 us in
+    // 8 parts).  An M-contiguous A takes 8 parts (the register-staged plan it
+    // replaces had up to 8).
+    const int64_t t64 = cdiv(M, 64) * cdiv(N, 64), KT = cdiv(K, 32);
+    const bool few = 4 * t64 <= cus, deep = rag32 && t64 < cus && K >= 8192;
+    int64_t sp = few && a_kmajor ? cus / (t64 > 0 ? t64 : 1) : kMaxSplit32;
     if (sp > kMaxSplit32) sp = kMaxSplit32;
     if (sp > KT / 4) sp = KT / 4;
-    if (4 * t64 <= cus && sp >= 2) {
-      plan.cfg = TILE32_DMA_SPLIT;
+    if ((few || deep) && sp >= 2) {
+      plan.cfg = rag32 ? TILE32_RAG_SPLIT : TILE32_DMA_SPLIT;
       p.split = (int)sp;
     }
   }
@@ -721,8 +748,8 @@ static int gemm_run(int transA, int transB, int64_t M, int64_t N, int64_t K, int
   size_t part_bytes = 0;
   int counters = 0;
   gemm_split_needs(plan, &part_bytes, &counters);
-  if (part_bytes > 0 && is_mid(plan.cfg) && st != nullptr) {
-    // A mid-size split is only a matter of speed, so a call being captured
+  if (part_bytes > 0 && split_optional(plan.cfg) && st != nullptr) {
+    // These splits are only a matter of speed, so a call being captured
     // into a graph goes without one: nothing is allocated or waited for.
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
@@ -773,7 +800,7 @@ int sf_gemm_plan(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
   char extra[64] = "";
   if (!plan.noop && plan.p.split > 0)
     snprintf(extra, sizeof(extra), "%s split%s %dx%d", plan.p.persist > 0 ? " persistent" : "",
-             is_mid(plan.cfg) ? "" : "-tail",
+             split_optional(plan.cfg) ? "" : "-tail",
              plan.p.tiles_m * plan.p.tiles_n - plan.p.full_tiles, plan.p.split);
   else if (!plan.noop && plan.p.persist > 0)
     snprintf(extra, sizeof(extra), " persistent");

@@ -19,19 +19,37 @@ static int launch32_t(int cfg, const GemmParams& p, unsigned gx, unsigned gy, hi
     case TILE_GENERIC:
       hipLaunchKernelGGL((gemm32_kernel<64, 64, 2, 2, KM, false, AKM>), g, dim3(256), 0, st, p);
       break;
+    case TILE32_DMA:
+      if constexpr (AKM) {
+        if (p.K % 64 == 0) {
+          hipLaunchKernelGGL((gemm32dma_kernel<64, 64, AKM, KM, 2, 2, 4, false>), g, dim3(512), 0, st, p);
+          break;
+        }
+      }
+      hipLaunchKernelGGL((gemm32dma_kernel<64, 64, AKM, KM, 2, 2>), g, dim3(512), 0, st, p);
+      break;
+    case TILE32_DMA_SPLIT:
+      if constexpr (AKM) {
+        if (p.K % 32 == 0) {
+          hipLaunchKernelGGL((gemm32dma_kernel<64, 64, AKM, KM, 3, 1, 4, false>), g, dim3(256), 0, st, p);
+          break;
+        }
+      }
+      hipLaunchKernelGGL((gemm32dma_kernel<64, 64, AKM, KM, 3, 1>), g, dim3(256), 0, st, p);
+      break;
+    case TILE32_RAG:
+      hipLaunchKernelGGL((gemm32dma_kernel<64, 64, AKM, KM, 2, 2, 1>), g, dim3(512), 0, st, p);
+      break;
+    case TILE32_RAG_SPLIT:
+      hipLaunchKernelGGL((gemm32dma_kernel<64, 64, AKM, KM, 3, 1, 1>), g, dim3(256), 0, st, p);
+      break;
     case TILE32_SMALL1:
     case TILE32_SMALL2:
-    case TILE32_DMA:
-    case TILE32_DMA_SPLIT:
       if constexpr (AKM) {
         if (cfg == TILE32_SMALL1)
           hipLaunchKernelGGL((gemm32small_kernel<1, KM, 4>), g, dim3(256), 0, st, p);
-        else if (cfg == TILE32_SMALL2)
-          hipLaunchKernelGGL((gemm32small_kernel<2, KM, 8>), g, dim3(512), 0, st, p);
-        else if (cfg == TILE32_DMA)
-          hipLaunchKernelGGL((gemm32dma_kernel<64, 64, KM, 2, 2>), g, dim3(512), 0, st, p);
         else
-          hipLaunchKernelGGL((gemm32dma_kernel<64, 64, KM, 3, 1>), g, dim3(256), 0, st, p);
+          hipLaunchKernelGGL((gemm32small_kernel<2, KM, 8>), g, dim3(512), 0, st, p);
         break;
       }
       return fail(SF_ERR_INVALID_ARG, "tile config %d needs a K-contiguous A", cfg);
@@ -42,8 +60,8 @@ static int launch32_t(int cfg, const GemmParams& p, unsigned gx, unsigned gy, hi
 }
 
 int launch_gemm32(bool a_kmajor, bool b_kmajor, int cfg, const GemmParams& p, int64_t batch, hipStream_t st) {
-  if (p.split > kMaxSplit32 || (p.split > 0 && batch != 1) || (cfg == TILE32_DMA && p.split > 0) ||
-      (cfg == TILE32_DMA && (p.K / 32) % 2 != 0))
+  if (p.split > kMaxSplit32 || (p.split > 0 && batch != 1) ||
+      ((cfg == TILE32_DMA || cfg == TILE32_RAG) && p.split > 0))
     return fail(SF_ERR_INVALID_ARG, "fp32 plan: split %d / batch %lld / K %d do not fit tile config %d", p.split,
                 (long long)batch, p.K, cfg);
   const unsigned gx = static_cast<unsigned>(p.tiles_m) * static_cast<unsigned>(p.tiles_n) *

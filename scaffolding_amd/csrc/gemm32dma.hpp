@@ -3,8 +3,13 @@
 //
 //   C[b] = epi(alpha * A[b] . op(B[b]) (+ bias)) (+ R[b])     row-major, fp32
 //
-// A is M x K (K-contiguous); B is N x K (K-contiguous, "NT": x . W^T) or
-// K x N (N-contiguous, "NN": A . B).  K % 32 == 0, rows 16-byte aligned.
+// A is M x K (K-contiguous) or stored K x M (M-contiguous: the product uses
+// its transpose, dW = dY^T X); B is N x K (K-contiguous, "NT": x . W^T) or
+// K x N (N-contiguous, "NN": A . B).  Any K: chunks past it are sent out of
+// the buffer's range (zeros).  CE: floats a lane loads at once, 4 (rows
+// 16-byte aligned) or 1 (rows and sizes of any float alignment: four times
+// the load instructions, which the MFMAs still cover).  TAIL = false: K a
+// multiple of 32 KG, without the per-slice checks (1024^3 NN 22.1 -> 21.4 us).
 //
 // Why.  An fp32 MFMA slice (32 k) of a 64 x 64 tile is 32 MFMAs per wave,
 // about 1000 cycles, shorter than a global-load round trip under load; the
@@ -12,6 +17,15 @@
 // every one.  Here buffer_load_dwordx4 ... lds moves each slice straight
 // into LDS (no VGPRs, no ds_write) NSTG - 1 slices ahead of the one the
 // MFMAs consume.
+//
+// Measured on one MI355X (us, register-staged gemm32.hpp -> this kernel):
+//   TN 1024 x 1024 x 2048             61.8 -> 39.1  (110 TFLOP/s)
+//   TN 1920 x 1920 x 2048            174   -> 133   (114 TFLOP/s)
+//   NN 1000^3 (K no multiple of 32)   32.1 -> 22.3  (90 TFLOP/s)
+//   CE == 1, element-wise loads before:
+//   NT 2048 x 2048 x 2050            286   -> 177   (97 TFLOP/s)
+//   NN 2001 x 2003 x 1001            130   -> 89    (90 TFLOP/s)
+//   NT 33 x 1025 x 4097, 8 parts     136   -> 25.2
 //
 // Work decomposition: 256 threads, waves 2 x 2 of (BM/2) x (BN/2), MFMA X
 // operand from B, Y from A; lane l ends with fragment rows 4 (l / 16) + q of
@@ -27,7 +41,8 @@
 //     reads, which hold k = 4 g .. 4 g + 3, one per step.  A direct load
 //     fills 8 rows (lane l: row l >> 3, slot l & 7, chunk (l & 7) ^ (l >> 3)).
 //     Fragment i of a wave holds rows (columns of C) wn WN + 16 i + r.
-//   N-contiguous B: k-row k = BN floats.  Fragment i of a wave's X operand
+//   N-contiguous B (an M-contiguous A likewise, with BM, FM and m): k-row k =
+//     BN floats.  Fragment i of a wave's X operand
 //     holds columns n = wn WN + FN r + i (r = fragment row), so at step s
 //     lane l reads the FN consecutive floats B[k][wn WN + FN (l & 15) + i]
 //     of k-row k = 4 g + s in one ds_read (b128 at FN = 4, b64 at FN = 2)
@@ -73,7 +88,12 @@ __device__ __forceinline__ void lds_wait_all() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int BM, int BN, bool B_KMAJOR, int NSTG, int KG = 1>
+// Four floats at any 4-byte alignment (one global_store_dwordx4).
+struct __attribute__((packed, aligned(4))) Float4u {
+  f32x4 v;
+};
+
+template <int BM, int BN, bool A_KMAJOR, bool B_KMAJOR, int NSTG, int KG = 1, int CE = 4, bool TAIL = true>
 __global__ __launch_bounds__(256 * KG) void gemm32dma_kernel(GemmParams p) {
   constexpr int NT = 256;  // threads of one k-group
   constexpr int BK = 32;
@@ -82,9 +102,13 @@ __global__ __launch_bounds__(256 * KG) void gemm32dma_kernel(GemmParams p) {
   constexpr int A_BYTES = BM * BK * 4;
   constexpr int B_BYTES = BN * BK * 4;
   constexpr int SLOT = A_BYTES + B_BYTES;
-  constexpr int LA = A_BYTES / 1024 / 4;  // direct loads per wave per slice, A
-  constexpr int LB = B_BYTES / 1024 / 4;  // and B
+  constexpr int LD_BYTES = 256 * CE;          // bytes of one direct load
+  constexpr int LA = A_BYTES / LD_BYTES / 4;  // direct loads per wave per slice, A
+  constexpr int LB = B_BYTES / LD_BYTES / 4;  // and B
   constexpr int L = LA + LB;
+  static_assert(CE == 4 || CE == 1, "16- or 4-byte loads");
+  static_assert(A_KMAJOR || FM == 2 || FM == 4, "M-contiguous A reads 2 or 4 rows per lane");
+  static_assert(BM <= 64 * CE && BN <= 64 * CE, "a load covers whole k-rows");
   static_assert(LA >= 1 && LB >= 1, "each wave loads part of both operands");
   static_assert(B_KMAJOR || FN == 2 || FN == 4, "N-contiguous B reads 2 or 4 columns per lane");
   static_assert(NSTG >= 2 && L * (NSTG - 2) < 64, "vmcnt holds at most 63");
@@ -111,69 +135,93 @@ __global__ __launch_bounds__(256 * KG) void gemm32dma_kernel(GemmParams p) {
   const float* B = static_cast<const float*>(p.B) + b * p.sB;
   const int M = p.M, N = p.N, K = p.K;
 
-  // This k-group's slices [kt0, kt1): with two groups the host keeps the
-  // slice count even, so both run the same number of iterations (and
-  // workgroup barriers).
-  const int KTall = K / BK;
+  // This k-group's slices [kt0, kt1): with two groups the count is rounded
+  // up to even (a slice past K is all zeros), so both run the same number of
+  // iterations (and workgroup barriers).
+  const int KTall = (K + BK * KG - 1) / (BK * KG) * KG;
   const int kt0 = part >= 0 ? KTall * part / p.split : kg * (KTall / KG);
   const int kt1 = part >= 0 ? KTall * (part + 1) / p.split : kt0 + KTall / KG;
   const int last = kt1 - 1;
 
-  // Buffer resources over this batch entry's rows (the host keeps them
-  // under 2^31 bytes).  Rows past M (N) are clamped to the last row (their
-  // products reach no stored output); for an N-contiguous B, columns past N
-  // read the next row or, past the buffer, zeros (likewise unstored).
-  const __amdgpu_buffer_rsrc_t rA =
-      __builtin_amdgcn_make_buffer_rsrc((void*)A, (short)0, (int)((uint32_t)M * (uint32_t)p.lda * 4u), 0x00020000);
+  // Buffer resources over this batch entry's rows (the host keeps them, and
+  // 64 k-rows more, under 2^31 bytes).  Rows past M (N) of a K-contiguous
+  // operand are clamped to the last row (their products reach no stored
+  // output); k past K, and columns past the edge of an operand with k-rows,
+  // are out of range: zeros.  (k-rows past K lie past the buffer's end.)
+  constexpr uint32_t OOB = 0x80000000u;
+  const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)A, (short)0, (int)((uint32_t)(A_KMAJOR ? M : K) * (uint32_t)p.lda * 4u), 0x00020000);
   const __amdgpu_buffer_rsrc_t rB = __builtin_amdgcn_make_buffer_rsrc(
       (void*)B, (short)0, (int)((uint32_t)(B_KMAJOR ? N : K) * (uint32_t)p.ldb * 4u), 0x00020000);
+  // K-contiguous: load w covers RPL = 8 (CE == 4) or 2 rows of 32 floats.
+  // kcol: the lane's k within its row's slice.
+  auto km_row = [&](int w) { return CE == 4 ? w * 8 + (lane >> 3) : w * 2 + (lane >> 5); };
+  auto km_col = [&](int w) {
+    const int r = km_row(w) & 7;
+    return CE == 4 ? ((lane & 7) ^ r) * 4 : ((((lane & 31) >> 2) ^ r) * 4 + (lane & 3));
+  };
+  auto km_off = [&](int w, int r0, int rows, int64_t ld) {
+    const int r = r0 + km_row(w) < rows ? r0 + km_row(w) : rows - 1;
+    return (uint32_t)r * (uint32_t)ld * 4u + (uint32_t)(km_col(w) * 4);
+  };
+  // k-rows of W floats: a load covers 64 CE / W of them; F fragments per
+  // wave decide the swap of row halves.
+  auto mn_off = [&](auto w_c, auto f_c, int w, int c0, int cols, int64_t ld) {
+    constexpr int W = decltype(w_c)::value, F = decltype(f_c)::value;
+    constexpr int LPR = W / CE;  // lanes per k-row
+    const int kr = w * (64 / LPR) + lane / LPR;
+    const int slot = (lane % LPR) * CE / 4;  // 16-byte slot
+    const int chunk = F == 2 ? slot ^ (8 * ((kr >> 2) & 1)) : slot;
+    const int col = c0 + chunk * 4 + (CE == 4 ? 0 : (lane & 3));
+    return col < cols ? (uint32_t)kr * (uint32_t)ld * 4u + (uint32_t)(col * 4) : OOB;
+  };
+  constexpr std::integral_constant<int, BM> bm_c{};
+  constexpr std::integral_constant<int, BN> bn_c{};
+  constexpr std::integral_constant<int, FM> fm_c{};
+  constexpr std::integral_constant<int, FN> fn_c{};
   uint32_t voa[LA], vob[LB];
 #pragma unroll
-  for (int i = 0; i < LA; ++i) {
-    const int r = (wave * LA + i) * 8 + (lane >> 3);
-    const int gm = m0 + r < M ? m0 + r : M - 1;
-    voa[i] = (uint32_t)gm * (uint32_t)p.lda * 4u + (uint32_t)(((lane & 7) ^ (r & 7)) * 16);
-  }
+  for (int i = 0; i < LA; ++i)
+    voa[i] = A_KMAJOR ? km_off(wave * LA + i, m0, M, p.lda) : mn_off(bm_c, fm_c, wave * LA + i, m0, M, p.lda);
 #pragma unroll
-  for (int i = 0; i < LB; ++i) {
-    if constexpr (B_KMAJOR) {
-      const int r = (wave * LB + i) * 8 + (lane >> 3);
-      const int gn = n0 + r < N ? n0 + r : N - 1;
-      vob[i] = (uint32_t)gn * (uint32_t)p.ldb * 4u + (uint32_t)(((lane & 7) ^ (r & 7)) * 16);
-    } else {
-      // k-rows of BN floats: RPL k-rows per load, lane l on k-row l / CPR,
-      // slot l % CPR.
-      constexpr int CPR = BN / 4;    // 16-byte chunks per k-row
-      constexpr int RPL = 64 / CPR;  // k-rows per load
-      const int kr = (wave * LB + i) * RPL + lane / CPR;
-      const int slot = lane % CPR;
-      const int chunk = FN == 2 ? slot ^ (8 * ((kr >> 2) & 1)) : slot;
-      vob[i] = (uint32_t)kr * (uint32_t)p.ldb * 4u + (uint32_t)(n0 * 4 + chunk * 16);
-    }
-  }
+  for (int i = 0; i < LB; ++i)
+    vob[i] = B_KMAJOR ? km_off(wave * LB + i, n0, N, p.ldb) : mn_off(bn_c, fn_c, wave * LB + i, n0, N, p.ldb);
   // Fill u: slice min(u, last) into slot u % NSTG (the k offset of a
-  // K-contiguous operand goes in the scalar offset; an N-contiguous B moves
-  // by 32 k-rows).
+  // K-contiguous operand goes in the scalar offset; one with k-rows moves by
+  // 32 of them).
   // (The lane offsets come in as pointer arguments: a lambda that captures
   // an array whose length depends on the template parameters leaves the
   // kernel's host stub undefined with this compiler.)
+  auto load = [&](__amdgpu_buffer_rsrc_t r, uint8_t* dst, uint32_t vo, int so) {
+    if constexpr (CE == 4) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)dst, 16, vo, so, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)dst, 4, vo, so, 0, 0);
+  };
   auto issue = [&](int u, const uint32_t* va, const uint32_t* vb) {
     const int s = u % NSTG;
     const int t = u < last ? u : last;
     uint8_t* sa = ring + s * SLOT;
     uint8_t* sb = sa + A_BYTES;
+    const bool tail = TAIL && (t + 1) * BK > K;           // uniform
+    const int so = !TAIL || t * BK < K ? t * BK * 4 : 0;  // never past the buffer: its range check subtracts it
 #pragma unroll
-    for (int i = 0; i < LA; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, (lds_ptr_t)(sa + (wave * LA + i) * 1024), 16, va[i], t * BK * 4,
-                                               0, 0);
+    for (int i = 0; i < LA; ++i) {
+      uint32_t o = va[i];
+      if constexpr (A_KMAJOR) {
+        if (tail && t * BK + km_col(wave * LA + i) >= K) o = OOB;
+      } else {
+        o += (uint32_t)(t * BK) * (uint32_t)p.lda * 4u;
+      }
+      load(rA, sa + (wave * LA + i) * LD_BYTES, o, A_KMAJOR ? so : 0);
+    }
 #pragma unroll
     for (int i = 0; i < LB; ++i) {
-      if constexpr (B_KMAJOR)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, (lds_ptr_t)(sb + (wave * LB + i) * 1024), 16, vb[i],
-                                                 t * BK * 4, 0, 0);
-      else
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, (lds_ptr_t)(sb + (wave * LB + i) * 1024), 16,
-                                                 vb[i] + (uint32_t)(t * BK) * (uint32_t)p.ldb * 4u, 0, 0, 0);
+      uint32_t o = vb[i];
+      if constexpr (B_KMAJOR) {
+        if (tail && t * BK + km_col(wave * LB + i) >= K) o = OOB;
+      } else {
+        o += (uint32_t)(t * BK) * (uint32_t)p.ldb * 4u;
+      }
+      load(rB, sb + (wave * LB + i) * LD_BYTES, o, B_KMAJOR ? so : 0);
     }
   };
 
@@ -194,19 +242,38 @@ __global__ __launch_bounds__(256 * KG) void gemm32dma_kernel(GemmParams p) {
   const int sw = lane & 7;
   const uint32_t xcol = (uint32_t)((wn * WN + FN * (lane & 15)) * 4);
   const uint32_t xrow = (uint32_t)(4 * g * BN * 4) + (FN == 2 ? (xcol ^ (uint32_t)(128 * (g & 1))) : xcol);
+  const uint32_t ycol = (uint32_t)((wm * WM + FM * (lane & 15)) * 4);
+  const uint32_t yrow = (uint32_t)(4 * g * BM * 4) + (FM == 2 ? (ycol ^ (uint32_t)(128 * (g & 1))) : ycol);
 
   // Fragments of one 16-k step pair (kk): Y from A, X from B by step s.
   struct Frags {
     f32x4 y[FM];
     float x[4][FN];
   };
-  constexpr int NR = FM + (B_KMAJOR ? FN : 4);  // LDS reads per kk
+  constexpr int NR = (A_KMAJOR ? FM : 4) + (B_KMAJOR ? FN : 4);  // LDS reads per kk
   auto read = [&](uint32_t sa, uint32_t sb, int kk, Frags& f) {
     const uint32_t cs = (uint32_t)(((kk * 4 + g) ^ sw) << 4);
-    static_for<FM>([&](auto j_c) {
-      constexpr int J = decltype(j_c)::value;
-      f.y[J] = __builtin_bit_cast(f32x4, ds_read16<J * 16 * 128>(sa + fa + cs));
-    });
+    if constexpr (A_KMAJOR) {
+      static_for<FM>([&](auto j_c) {
+        constexpr int J = decltype(j_c)::value;
+        f.y[J] = __builtin_bit_cast(f32x4, ds_read16<J * 16 * 128>(sa + fa + cs));
+      });
+    } else {
+      // Step s: A[k = kk*16 + 4g + s][wm*WM + FM (l & 15) + j], all j.
+      const uint32_t ya = sa + yrow + (uint32_t)(kk * 16 * BM * 4);
+      static_for<4>([&](auto s_c) {
+        constexpr int S = decltype(s_c)::value;
+        if constexpr (FM == 4) {
+          const f32x4 v = __builtin_bit_cast(f32x4, ds_read16<S * BM * 4>(ya));
+#pragma unroll
+          for (int j = 0; j < 4; ++j) f.y[j][S] = v[j];
+        } else {
+          const uint64_t v = ds_read8<S * BM * 4>(ya);
+          f.y[0][S] = __builtin_bit_cast(float, (uint32_t)v);
+          f.y[1][S] = __builtin_bit_cast(float, (uint32_t)(v >> 32));
+        }
+      });
+    }
     if constexpr (B_KMAJOR) {
       static_for<FN>([&](auto i_c) {
         constexpr int I = decltype(i_c)::value;
@@ -300,7 +367,8 @@ __global__ __launch_bounds__(256 * KG) void gemm32dma_kernel(GemmParams p) {
   // Epilogue, in runs of 4 consecutive columns per lane: K-contiguous B,
   // run c = fragment c's rows 4g..4g+3; N-contiguous B, run c = columns
   // wn*WN + 4 FN g + 4c + e, element e of run c from fragment (4c+e) % FN,
-  // row (4c+e) / FN.
+  // row (4c+e) / FN.  Fragment j's rows of C: 16 j + l % 16, or with an
+  // M-contiguous A FM (l % 16) + j.
   float* C = static_cast<float*>(p.C) + b * p.sC;
   const bool has_bias = epi_has_bias(p.epi);
   const int act = epi_act(p.epi);
@@ -321,7 +389,7 @@ __global__ __launch_bounds__(256 * KG) void gemm32dma_kernel(GemmParams p) {
       }
 #pragma unroll
       for (int j = 0; j < FM; ++j) {
-        const int m = m0 + wm * WM + j * 16 + (lane & 15);
+        const int m = m0 + wm * WM + (A_KMAJOR ? j * 16 + (lane & 15) : FM * (lane & 15) + j);
         if (m < M && n < N) {
           float v[4];
 #pragma unroll
@@ -335,7 +403,10 @@ __global__ __launch_bounds__(256 * KG) void gemm32dma_kernel(GemmParams p) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] += r[e];
           }
-          Store4<float>::run(C + (int64_t)m * p.ldc, n, N, vec_ok, v);
+          if (CE == 1 && n + 3 < N)
+            reinterpret_cast<Float4u*>(C + (int64_t)m * p.ldc + n)->v = f32x4{v[0], v[1], v[2], v[3]};
+          else
+            Store4<float>::run(C + (int64_t)m * p.ldc, n, N, vec_ok, v);
         }
       }
     }

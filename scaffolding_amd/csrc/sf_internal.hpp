@@ -41,7 +41,7 @@ enum TileCfg {
   TILE_128x128 = 2,  // fp32; 16-bit inputs with an fp32 output: 256 threads, waves 2x2 of 64x64
   TILE_256x64 = 3,   // 256 threads, waves 4x1 of 64x64 (narrow N, e.g. P.V)
   TILE_64x64 = 4,    // fp32 only
-  TILE_GENERIC = 5,  // fp32 or an fp32 output: 64x64, element-wise bounds-checked loads (any layout)
+  TILE_GENERIC = 5,  // fp32 past 2 GiB, or an fp32 output: 64x64, element-wise bounds-checked loads (any layout)
   TILE_SKINNY = 6,   // M <= 16 stream kernel
   TILE_NT_BIG = 7,   // 256x256 NT, 8-wave ping-pong, direct-to-LDS (gemm16nt_pp.hpp)
   TILE_SKINNY_LINE = 8,  // M <= 16, K in {2048, 4096, 8192}: row-segment stream (skinny16l)
@@ -57,9 +57,14 @@ enum TileCfg {
   TILE_MID_64 = 15,    // 64x64, direct-to-LDS ring of 3, three workgroups per CU
   TILE_MID_32 = 16,    // 32x64 (NT), direct-to-LDS ring of 4, three workgroups per CU
   TILE_RAG_128 = 17,   // 128x128, register-staged loads at any 2-byte alignment
-  TILE_RAG_64 = 18     // 64x64, likewise
+  TILE_RAG_64 = 18,    // 64x64, likewise
+  // fp32, operands at any 4-byte alignment (gemm32dma.hpp with 4-byte loads):
+  TILE32_RAG = 19,       // as TILE32_DMA
+  TILE32_RAG_SPLIT = 20  // as TILE32_DMA_SPLIT
 };
 const char* tile_name(int cfg);
+// Plans whose split may be left out (the unsplit kernel is the same one).
+inline bool split_optional(int cfg) { return (cfg >= TILE_MID_128 && cfg <= TILE_RAG_64) || cfg == TILE32_RAG_SPLIT; }
 inline bool is_mid(int cfg) { return cfg >= TILE_MID_128 && cfg <= TILE_RAG_64; }
 
 // One GEMM launch: batch entries [0, batch) of p, grid.y <= 65535 per call.
