@@ -130,9 +130,10 @@ int sf_set_test_hooks(int xcd_shift, int split_spins, int attn_parts);
  * M, N or batch == 0 is a no-op; K == 0 writes epi(0 (+ bias)).
  * The call is asynchronous on `stream`.  Some plans split tiles along k and
  * pass fp32 partials through a per-device workspace, allocated on first use
- * (see sf_gemm_noalloc).  On a stream that is being captured, mid-size 16-bit
- * problems (fewer than one 256 x 256 tile per CU) and unaligned operands run
- * without that split, so capturing them allocates nothing. */
+ * (see sf_gemm_noalloc).  On a stream that is being captured every problem
+ * runs without a split: the call allocates nothing and its graph holds no
+ * library memory, so replays need no ordering against other calls.  (A sum
+ * that the eager call splits may differ there in its last bits.) */
 int sf_gemm(int transA, int transB,
             int64_t M, int64_t N, int64_t K, int64_t batch,
             const void* A, int64_t lda, int64_t strideA,
@@ -164,8 +165,9 @@ int sf_gemm_add(int transA, int transB,
  * graph capture, tight serving loops, harnesses that forbid hipMalloc.  No
  * counterpart in the reference (cuBLAS keeps its workspace internally).
  *
- * Same arguments, rules, kernels and results (bit for bit) as sf_gemm.  Where
- * sf_gemm's plan splits tiles along k (it then allocates a per-device
+ * Same arguments, rules, kernels and results (bit for bit) as sf_gemm on a
+ * stream that is not being captured; captured, this call keeps the split.
+ * Where sf_gemm's plan splits tiles along k (it then allocates a per-device
  * workspace on first use), this entry point takes the fp32 partials and the
  * arrival counters from a fixed per-device scratch array of
  * SF_NOALLOC_SCRATCH_BYTES inside the library, which each GPU the library
@@ -209,7 +211,10 @@ int sf_gemm_plan(int transA, int transB,
  * autograd.py:819).  in_dtype in {F32, F16, BF16}; out_dtype is in_dtype or
  * F32; fp32 accumulation in an order fixed by the shape (results do not
  * vary between calls).  dim_size == 0 writes zeros.  Column sums over many
- * rows use the library's per-device workspace.  Asynchronous on `stream`. */
+ * rows use the library's per-device workspace; captured ones a second
+ * buffer of the device that is only for captured calls (of sf_sum_dim and
+ * the fused attention: replays of their graphs that overlap on one device
+ * race) and stays where it is once allocated.  Asynchronous on `stream`. */
 int sf_sum_dim(const void* x, void* out, int64_t outer, int64_t dim_size, int64_t inner,
                sf_dtype in_dtype, sf_dtype out_dtype, void* stream);
 
@@ -230,8 +235,8 @@ int sf_sum_dim(const void* x, void* out, int64_t outer, int64_t dim_size, int64_
  * sf_softmax_rows).  Any Sk >= 1.  When the last round of work items
  * (256 query rows of one batch entry) would leave most of the GPU idle,
  * those items are split over key ranges whose fp32 partials pass through
- * the library's per-device workspace (as sf_sum_dim's do) and are merged
- * by a second launch. */
+ * the library's per-device workspace (as sf_sum_dim's do, under capture
+ * too) and are merged by a second launch. */
 int sf_attention(const void* Q, int64_t ldq, int64_t strideQ,
                  const void* K, int64_t ldk, int64_t strideK,
                  const void* V, int64_t ldv, int64_t strideV,

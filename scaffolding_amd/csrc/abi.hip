@@ -212,7 +212,7 @@ static float big_cost(int64_t t256, int64_t K, bool can_split, int cus) {
 
 // Picks the 16-bit tile config and, for the mid-size kernels, the k split.
 static int choose_tile16(int64_t M, int64_t N, int64_t K, int64_t batch, bool vec, bool small, bool a_kmajor,
-                         bool b_kmajor, bool f32_out, int cus, int* split) {
+                         bool b_kmajor, bool f32_out, bool may_split, int cus, int* split) {
   *split = 0;
   // K-contiguous operands need whole 16-byte chunks along k.
   const bool kvec = vec && (K % 8 == 0 || (!a_kmajor && !b_kmajor));
@@ -234,7 +234,7 @@ static int choose_tile16(int64_t M, int64_t N, int64_t K, int64_t batch, bool ve
     const bool k_ok = K >= 128 && (K % 128 == 0 || (!a_kmajor && !b_kmajor));
     if (k_ok && N > 64 && M > 64) {
       if (t256 >= cus) return TILE_NT_BIG;
-      const bool can_split = batch == 1 && K >= 1024 && 16 * t256 >= cus;
+      const bool can_split = may_split && batch == 1 && K >= 1024 && 16 * t256 >= cus;
       // TT, TN with a ragged K whose split tiles fill the CUs exactly, and
       // parts with more CUs than the estimates below were fitted on keep the
       // split of the 256 x 256 kernel.
@@ -262,7 +262,7 @@ static int choose_tile16(int64_t M, int64_t N, int64_t K, int64_t batch, bool ve
     const int64_t t = tiles(c[i].bm, c[i].bn);
     for (int sp = 1; sp <= kMaxSplitMid; ++sp) {
       // parts of at least two slices, all resident together
-      if (sp > 1 && (batch != 1 || tt || KT < 2 * sp || t * sp > (int64_t)c[i].occ * cus)) break;
+      if (sp > 1 && (!may_split || batch != 1 || tt || KT < 2 * sp || t * sp > (int64_t)c[i].occ * cus)) break;
       const float us = mid_cost(c[i], M, N, K, batch, sp, cus);
       if (us < best) {
         best = us;
@@ -323,6 +323,14 @@ static int choose_tile32(int64_t M, int64_t N, int64_t K, int64_t batch, bool ve
 // from split_workspace_acquire to split_workspace_release, so calls from
 // several host threads enqueue their workspace launches one at a time and
 // each one's event wait sees the previous one's record.
+//
+// A stream that is being captured never touches that buffer: its replays
+// would run outside the ordering above and outlive the buffer's growth.
+// GEMMs are planned without a split then (gemm_run); attention and column
+// sums, whose partials need no counters, take the device's capture buffer,
+// which no eager call uses.  Growing it keeps the old buffers (graphs hold
+// their addresses; each is at least twice the one before, so together they
+// are no larger than the newest) until the process ends.
 // ---------------------------------------------------------------------
 struct SplitWorkspace {
   void* base = nullptr;
@@ -332,24 +340,71 @@ struct SplitWorkspace {
   hipStream_t last = nullptr;
   bool used = false;
   bool multi = false;  // split launches have come on more than one stream
+  void* capture_base = nullptr;
+  size_t capture_bytes = 0;  // of the newest capture buffer
+  size_t capture_total = 0;  // of all of them
 };
 static std::mutex g_ws_mu;
 static std::unordered_map<int, SplitWorkspace> g_ws;
 
+// The legacy stream cannot be captured (and asking about it while another
+// stream is would fail).
+static bool stream_capturing(hipStream_t st) {
+  if (st == nullptr) return false;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return cap != hipStreamCaptureStatusNone;
+}
+
+// While alive, this thread may allocate, free and synchronise although some
+// stream is being captured in the global or thread-local mode.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  bool on;
+  RelaxedCapture() : on(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+  ~RelaxedCapture() {
+    if (on) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+};
+
 static int split_workspace_acquire_locked(int dev, size_t part_bytes, int ncounters, hipStream_t st, float** ws,
                                           int** cnt);
+static int capture_workspace_locked(int dev, size_t part_bytes, float** ws);
 
 // On SF_OK the workspace lock stays held until split_workspace_release,
 // which the caller must then call (after its launch, whatever that
-// returned); on failure nothing stays locked.
-static int split_workspace_acquire(size_t part_bytes, int ncounters, hipStream_t st, float** ws, int** cnt) {
+// returned); on failure nothing stays locked.  `capturing`: st is being
+// captured (no counters then).
+static int split_workspace_acquire(size_t part_bytes, int ncounters, hipStream_t st, bool capturing, float** ws,
+                                   int** cnt) {
   int dev = 0;
   int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
   if (rc != SF_OK) return rc;
   g_ws_mu.lock();
-  rc = split_workspace_acquire_locked(dev, part_bytes, ncounters, st, ws, cnt);
+  *cnt = nullptr;
+  rc = capturing ? capture_workspace_locked(dev, part_bytes, ws)
+                 : split_workspace_acquire_locked(dev, part_bytes, ncounters, st, ws, cnt);
   if (rc != SF_OK) g_ws_mu.unlock();
   return rc;
+}
+
+static int capture_workspace_locked(int dev, size_t part_bytes, float** ws) {
+  SplitWorkspace& w = g_ws[dev];
+  if (part_bytes > w.capture_bytes) {
+    const size_t want = part_bytes > 2 * w.capture_bytes ? part_bytes : 2 * w.capture_bytes;
+    RelaxedCapture relaxed;
+    void* p = nullptr;
+    const int rc = check_hip(hipMalloc(&p, want), "hipMalloc (capture workspace)");
+    if (rc != SF_OK) return rc;
+    w.capture_base = p;
+    w.capture_bytes = want;
+    w.capture_total += want;
+  }
+  *ws = static_cast<float*>(w.capture_base);
+  return SF_OK;
 }
 
 static int split_workspace_acquire_locked(int dev, size_t part_bytes, int ncounters, hipStream_t st, float** ws,
@@ -363,6 +418,7 @@ static int split_workspace_acquire_locked(int dev, size_t part_bytes, int ncount
   if (part_bytes > w.part_bytes || ncounters > w.counters) {
     const size_t pb = part_bytes > w.part_bytes ? part_bytes : w.part_bytes;
     const int nc = ncounters > w.counters ? ncounters : w.counters;
+    RelaxedCapture relaxed;
     if (w.base != nullptr) {
       rc = check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize (split workspace)");
       if (rc != SF_OK) return rc;
@@ -402,8 +458,9 @@ static int split_workspace_acquire_locked(int dev, size_t part_bytes, int ncount
 // Records the event after the caller's launch (once split launches have
 // come on more than one stream) and releases the lock taken by
 // split_workspace_acquire.
-static int split_workspace_release(hipStream_t st) {
+static int split_workspace_release(hipStream_t st, bool capturing) {
   std::lock_guard<std::mutex> lk(g_ws_mu, std::adopt_lock);
+  if (capturing) return SF_OK;
   int dev = 0;
   int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
   if (rc != SF_OK) return rc;
@@ -459,12 +516,13 @@ int sf_set_test_hooks(int xcd_shift, int split_spins, int attn_parts) {
 namespace sf {
 
 // Validates sf_gemm's arguments and fills the launch plan (GemmPlan,
-// sf_internal.hpp).  Returns SF_OK with plan.noop = true for an empty
+// sf_internal.hpp), without a k split unless may_split.  Returns SF_OK with plan.noop = true for an empty
 // problem.  No HIP call before validation.
 int gemm_prepare(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_t batch, const void* A,
                  int64_t lda, int64_t strideA, const void* B, int64_t ldb, int64_t strideB, void* C, int64_t ldc,
                  int64_t strideC, sf_dtype ab_dtype, sf_dtype c_dtype, float alpha, const void* bias,
-                 sf_epilogue epi, const void* R, int64_t ldr, int64_t strideR, bool need_c, GemmPlan& plan) {
+                 sf_epilogue epi, const void* R, int64_t ldr, int64_t strideR, bool need_c, bool may_split,
+                 GemmPlan& plan) {
   g_err[0] = 0;
   plan.noop = false;
   if (!valid_dtype(ab_dtype) || !valid_dtype(c_dtype))
@@ -552,7 +610,8 @@ int gemm_prepare(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
     const bool small = (a_kmajor ? M : K) * lda * 2 < (int64_t(1) << 31) &&
                        (b_kmajor ? N : K) * ldb * 2 < (int64_t(1) << 31);
     plan.fp32 = false;
-    plan.cfg = choose_tile16(M, N, K, batch, vec, small, a_kmajor, b_kmajor, c_dtype == SF_F32, cus, &mid_split);
+    plan.cfg = choose_tile16(M, N, K, batch, vec, small, a_kmajor, b_kmajor, c_dtype == SF_F32, may_split, cus,
+                             &mid_split);
   }
   // The row-segment skinny kernel addresses 64 rows of W with 32-bit offsets.
   if (plan.cfg == TILE_SKINNY_LINE && ldb * 2 * 64 >= (int64_t(1) << 31)) plan.cfg = TILE_SKINNY;
@@ -572,7 +631,8 @@ int gemm_prepare(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
   p.xcd_shift = 0;
   p.arrive_spins = kSplitArriveSpins;
   const bool rag32 = plan.fp32 && plan.cfg == TILE32_RAG;
-  if (plan.fp32 && batch == 1 && K >= 128 && (plan.cfg == TILE32_DMA || plan.cfg == TILE32_DMA_SPLIT || rag32)) {
+  if (plan.fp32 && may_split && batch == 1 && K >= 128 &&
+      (plan.cfg == TILE32_DMA || plan.cfg == TILE32_DMA_SPLIT || rag32)) {
     // LDS-DMA fp32 with at most CUs / 4 tiles of 64 x 64 (K > 2048, past the
     // small-block kernel): split every tile along k, at most 8 parts of at
     // least 4 slices (64 x 4096 x 4096 NT: 37.9 us in 4 parts against
@@ -592,7 +652,7 @@ int gemm_prepare(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
       p.split = (int)sp;
     }
   }
-  if (plan.fp32 && batch == 1 && K >= 128 && (plan.cfg == TILE_128x128 || plan.cfg == TILE_64x64)) {
+  if (plan.fp32 && may_split && batch == 1 && K >= 128 && (plan.cfg == TILE_128x128 || plan.cfg == TILE_64x64)) {
     // fp32 with fewer 64 x 64 tiles than CUs: split every tile along k (each
     // part at least 4 slices of 32), on 128 x 128 tiles when that reaches
     // half the CUs, else on 64 x 64 tiles.  With at least one 64 x 64 tile
@@ -665,7 +725,7 @@ int gemm_prepare(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
     const int64_t T = (int64_t)p.tiles_m * p.tiles_n, R = T % cus, units = (K + 127) / 128;
     const bool can_persist = a_kmajor && T > cus && cus % kNumXcd == 0;  // NT, or NN (dX)
     const int64_t min_units = T <= R ? 2 : (can_persist && T < 3 * cus ? 10 : 32);
-    if (R > 0 && 2 * R <= cus && units >= min_units && (T - R) % kNumXcd == 0) {
+    if (may_split && R > 0 && 2 * R <= cus && units >= min_units && (T - R) % kNumXcd == 0) {
       int64_t sp = cus / R;
       if (sp > units) sp = units;
       if (T > R && units < 32 && sp > units / 5) sp = units / 5;
@@ -742,26 +802,25 @@ static int gemm_run(int transA, int transB, int64_t M, int64_t N, int64_t K, int
                     void* stream) {
   GemmPlan plan;
   int rc = gemm_prepare(transA, transB, M, N, K, batch, A, lda, strideA, B, ldb, strideB, C, ldc,
-                        strideC, ab_dtype, c_dtype, alpha, bias, epi, R, ldr, strideR, true, plan);
+                        strideC, ab_dtype, c_dtype, alpha, bias, epi, R, ldr, strideR, true, true, plan);
   if (rc != SF_OK || plan.noop) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   size_t part_bytes = 0;
   int counters = 0;
   gemm_split_needs(plan, &part_bytes, &counters);
-  if (part_bytes > 0 && split_optional(plan.cfg) && st != nullptr) {
-    // These splits are only a matter of speed, so a call being captured
-    // into a graph goes without one: nothing is allocated or waited for.
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
-      plan.p.split = 0;
-      part_bytes = 0;
-    }
+  if (part_bytes > 0 && stream_capturing(st)) {
+    // A graph may not hold the shared workspace (see SplitWorkspace): the
+    // best plan without a split, nothing allocated or waited for.
+    rc = gemm_prepare(transA, transB, M, N, K, batch, A, lda, strideA, B, ldb, strideB, C, ldc, strideC, ab_dtype,
+                      c_dtype, alpha, bias, epi, R, ldr, strideR, true, false, plan);
+    if (rc != SF_OK) return rc;
+    part_bytes = 0;
   }
   if (part_bytes == 0) return gemm_launch_plan(plan, batch, ab_dtype, c_dtype, st);
-  rc = split_workspace_acquire(part_bytes, counters, st, &plan.p.ws, &plan.p.counters);
+  rc = split_workspace_acquire(part_bytes, counters, st, false, &plan.p.ws, &plan.p.counters);
   if (rc != SF_OK) return rc;
   rc = gemm_launch_plan(plan, batch, ab_dtype, c_dtype, st);
-  const int rc2 = split_workspace_release(st);
+  const int rc2 = split_workspace_release(st, false);
   return rc != SF_OK ? rc : rc2;
 }
 
@@ -795,7 +854,7 @@ int sf_gemm_plan(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
   buf[0] = 0;
   GemmPlan plan;
   int rc = gemm_prepare(transA, transB, M, N, K, batch, A, lda, strideA, B, ldb, strideB, C, ldc,
-                        strideC, ab_dtype, c_dtype, alpha, bias, epi, nullptr, 0, 0, false, plan);
+                        strideC, ab_dtype, c_dtype, alpha, bias, epi, nullptr, 0, 0, false, true, plan);
   if (rc != SF_OK) return rc;
   char extra[64] = "";
   if (!plan.noop && plan.p.split > 0)
@@ -884,11 +943,12 @@ static int attn_wide_run(const AttnShape& a, const AttnMask& m, float scale, sf_
   if (sp.parts == 0) return launch_attention_wide(a, m, scale, dtype, sp, nullptr, st);
   float* ws = nullptr;
   int* cnt = nullptr;
+  const bool cap = stream_capturing(st);
   int rc = split_workspace_acquire((size_t)(sp.items - sp.full) * (size_t)sp.parts * attn_wide_part_bytes(a.D), 0, st,
-                                   &ws, &cnt);
+                                   cap, &ws, &cnt);
   if (rc != SF_OK) return rc;
   rc = launch_attention_wide(a, m, scale, dtype, sp, ws, st);
-  const int rc2 = split_workspace_release(st);
+  const int rc2 = split_workspace_release(st, cap);
   return rc != SF_OK ? rc : rc2;
 }
 
@@ -916,10 +976,12 @@ int sf_attention_heads(const void* Q, int64_t ldq, int64_t strideQ, int64_t head
   if (sp.parts == 0) return launch_attention(a, scale, dtype, sp, nullptr, st);
   float* ws = nullptr;
   int* cnt = nullptr;
-  rc = split_workspace_acquire((size_t)(sp.items - sp.full) * (size_t)sp.parts * kAttnPartBytes, 0, st, &ws, &cnt);
+  const bool cap = stream_capturing(st);
+  rc = split_workspace_acquire((size_t)(sp.items - sp.full) * (size_t)sp.parts * kAttnPartBytes, 0, st, cap, &ws,
+                               &cnt);
   if (rc != SF_OK) return rc;
   rc = launch_attention(a, scale, dtype, sp, ws, st);
-  const int rc2 = split_workspace_release(st);
+  const int rc2 = split_workspace_release(st, cap);
   return rc != SF_OK ? rc : rc2;
 }
 
@@ -1026,10 +1088,11 @@ int sf_sum_dim(const void* x, void* out, int64_t outer, int64_t dim_size, int64_
   if (S == 1) return launch_sum_dim(x, out, outer, dim_size, inner, in_dtype, out_dtype, nullptr, 1, st);
   float* ws = nullptr;
   int* cnt = nullptr;
-  int rc = split_workspace_acquire((size_t)S * (size_t)outer * (size_t)inner * sizeof(float), 0, st, &ws, &cnt);
+  const bool cap = stream_capturing(st);
+  int rc = split_workspace_acquire((size_t)S * (size_t)outer * (size_t)inner * sizeof(float), 0, st, cap, &ws, &cnt);
   if (rc != SF_OK) return rc;
   rc = launch_sum_dim(x, out, outer, dim_size, inner, in_dtype, out_dtype, ws, S, st);
-  const int rc2 = split_workspace_release(st);
+  const int rc2 = split_workspace_release(st, cap);
   return rc != SF_OK ? rc : rc2;
 }
 
@@ -1352,6 +1415,7 @@ int sf_workspace_bytes(int device, size_t* bytes) {
   for (auto& kv : g_ws) {
     if (device >= 0 && kv.first != device) continue;
     if (kv.second.base != nullptr) total += kv.second.part_bytes + (size_t)kv.second.counters * sizeof(int);
+    total += kv.second.capture_total;
   }
   *bytes = total;
   return SF_OK;

@@ -66,7 +66,7 @@ extern "C" int sf_gemm_noalloc(int transA, int transB, int64_t M, int64_t N, int
                                sf_dtype c_dtype, float alpha, const void* bias, sf_epilogue epi, void* stream) {
   GemmPlan plan;
   int rc = gemm_prepare(transA, transB, M, N, K, batch, A, lda, strideA, B, ldb, strideB, C, ldc, strideC,
-                        ab_dtype, c_dtype, alpha, bias, epi, nullptr, 0, 0, true, plan);
+                        ab_dtype, c_dtype, alpha, bias, epi, nullptr, 0, 0, true, true, plan);
   if (rc != SF_OK || plan.noop) return rc;
   size_t part_bytes = 0;
   int counters = 0;

@@ -89,11 +89,13 @@ struct GemmPlan {
   bool noop;  // an empty problem: nothing to launch
 };
 // Validates sf_gemm's arguments (R: residual of sf_gemm_add or NULL;
-// need_c: C must be non-NULL) and fills `plan`; no HIP call.
+// need_c: C must be non-NULL; may_split: whether the plan may cut tiles
+// along k) and fills `plan`; no HIP call.
 int gemm_prepare(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_t batch, const void* A,
                  int64_t lda, int64_t strideA, const void* B, int64_t ldb, int64_t strideB, void* C, int64_t ldc,
                  int64_t strideC, sf_dtype ab_dtype, sf_dtype c_dtype, float alpha, const void* bias,
-                 sf_epilogue epi, const void* R, int64_t ldr, int64_t strideR, bool need_c, GemmPlan& plan);
+                 sf_epilogue epi, const void* R, int64_t ldr, int64_t strideR, bool need_c, bool may_split,
+                 GemmPlan& plan);
 // The split plan's workspace: fp32 partials (*part_bytes, 0 without a
 // split) followed by *counters ints that must be zero at launch.
 void gemm_split_needs(const GemmPlan& plan, size_t* part_bytes, int* counters);
