@@ -129,8 +129,8 @@ int sf_set_test_hooks(int xcd_shift, int split_spins, int attn_parts);
  *
  * M, N or batch == 0 is a no-op; K == 0 writes epi(0 (+ bias)).
  * The call is asynchronous on `stream`.  Some plans split tiles along k and
- * pass fp32 partials through a per-device workspace, allocated on first use
- * (see sf_gemm_noalloc).  On a stream that is being captured every problem
+ * pass fp32 partials through a workspace, allocated on a stream's first use
+ * of one (see sf_workspace_bytes, sf_gemm_noalloc).  On a stream that is being captured every problem
  * runs without a split: the call allocates nothing and its graph holds no
  * library memory, so replays need no ordering against other calls.  (A sum
  * that the eager call splits may differ there in its last bits.) */
@@ -409,12 +409,15 @@ int sf_free(void* ptr);
  * `device` for the allocation and restores the caller's device. */
 int sf_cache_alloc(int device, size_t nbytes, void** ptr, size_t* got_bytes);
 int sf_cache_free(int device, void* ptr, size_t nbytes);
-int sf_cache_empty(int device);          /* device < 0: every device */
+/* device < 0: every device.  Also gives back the split workspaces of the
+ * second and further streams (after a device synchronize). */
+int sf_cache_empty(int device);
 int sf_cache_stats(int device, size_t* pooled_bytes, size_t* live_bytes);
 int sf_cache_set_limit(size_t bytes_per_device);
-/* Bytes of the per-device workspace that split plans (sf_gemm, sf_sum_dim,
- * sf_attention) allocate on first use, on `device` (< 0: every device); 0
- * before any such call.  Diagnostic, no reference counterpart. */
+/* Bytes of the workspaces that split plans (sf_gemm, sf_sum_dim,
+ * sf_attention) allocate on first use, on `device` (< 0: every device): one
+ * for each of up to four streams (further ones share them) and one for
+ * captured calls; 0 before any such call.  Diagnostic, no reference counterpart. */
 int sf_workspace_bytes(int device, size_t* bytes);
 
 /* Copies; synchronous w.r.t. the host when stream is NULL. */

@@ -10,6 +10,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <unordered_map>
 #include <vector>
@@ -310,47 +311,75 @@ static int choose_tile32(int64_t M, int64_t N, int64_t K, int64_t batch, bool ve
 }
 
 // ---------------------------------------------------------------------
-// Per-device workspace of the split-tail GEMM: fp32 partial tiles and one
-// counter per split tile.  Counters start at zero (cleared by a kernel when
-// the buffer is created) and every split tile's last part resets its own,
-// so the buffer is ready for the next launch.  Launches on one stream are
-// ordered by the stream, and while every split launch has come on one
-// stream nothing else is done (an event record costs about 3 us of host
-// time per call).  The first split launch on a second stream synchronises
-// the device once; from then on an event is recorded after every split
-// launch and a launch on another stream first waits for it.  Growing the
-// buffer synchronises the device before freeing the old one.  The lock is held
-// from split_workspace_acquire to split_workspace_release, so calls from
-// several host threads enqueue their workspace launches one at a time and
-// each one's event wait sees the previous one's record.
+// Workspace of the split plans: fp32 partial tiles and one counter per split
+// tile.  Counters start at zero (cleared by a kernel when the buffer is
+// created) and every split tile's last part resets its own, so the buffer is
+// ready for the next launch.  Each device has kWsSlots buffers, and a stream
+// takes one that no other stream uses, so split launches on a few streams
+// overlap and the stream alone orders those on one buffer (an event record
+// costs about 3 us of host time per call).  Streams past the slots share the
+// least recently used ones: the first launch of a second stream on a buffer
+// synchronises the device once; from then on an event is recorded after
+// every launch on that buffer, and a launch on another stream first waits
+// for it.  sf_stream_destroy records the event for the stream it ends.
+// Growing a buffer synchronises the device before freeing the old one.  A
+// buffer's lock is held from split_workspace_acquire to
+// split_workspace_release, so host threads that share one enqueue their
+// launches one at a time and each one's event wait sees the previous one's
+// record.  sf_cache_empty gives back every buffer but the first.
 //
-// A stream that is being captured never touches that buffer: its replays
-// would run outside the ordering above and outlive the buffer's growth.
+// A stream that is being captured never touches these buffers: its replays
+// would run outside the ordering above and outlive a buffer's growth.
 // GEMMs are planned without a split then (gemm_run); attention and column
 // sums, whose partials need no counters, take the device's capture buffer,
 // which no eager call uses.  Growing it keeps the old buffers (graphs hold
 // their addresses; each is at least twice the one before, so together they
 // are no larger than the newest) until the process ends.
 // ---------------------------------------------------------------------
+constexpr int kWsSlots = 4;
+typedef uintptr_t StreamKey;
+constexpr StreamKey kNoStream = ~StreamKey(0);
+
 struct SplitWorkspace {
+  std::mutex mu;             // everything below but owner and tick
   void* base = nullptr;
   size_t part_bytes = 0;
   int counters = 0;
   hipEvent_t done = nullptr;
-  hipStream_t last = nullptr;
+  StreamKey last = kNoStream;  // stream of the latest launch
   bool used = false;
-  bool multi = false;  // split launches have come on more than one stream
+  bool multi = false;     // several streams share this buffer
+  bool recorded = false;  // `done` follows the latest launch
+  StreamKey owner = kNoStream;  // under g_ws_mu: the stream that last took the slot
+  uint64_t tick = 0;            // and when
+};
+struct DeviceWorkspaces {
+  SplitWorkspace slot[kWsSlots];
+  uint64_t tick = 0;
   void* capture_base = nullptr;
   size_t capture_bytes = 0;  // of the newest capture buffer
   size_t capture_total = 0;  // of all of them
 };
+// The map, slot owners and ticks, capture buffers.  Never held while a
+// slot's lock is taken.
 static std::mutex g_ws_mu;
-static std::unordered_map<int, SplitWorkspace> g_ws;
+static std::unordered_map<int, DeviceWorkspaces> g_ws;
+
+// A stream's identity: its handle, but hipStreamPerThread names another
+// stream in every thread and hipStreamLegacy the null one.
+static StreamKey stream_key(hipStream_t st) {
+  if (st == hipStreamPerThread) {
+    static std::atomic<StreamKey> next{1};
+    thread_local const StreamKey id = next.fetch_add(1, std::memory_order_relaxed);
+    return (id << 2) | 3;  // no pointer
+  }
+  return st == hipStreamLegacy ? 0 : reinterpret_cast<StreamKey>(st);
+}
 
 // The legacy stream cannot be captured (and asking about it while another
 // stream is would fail).
 static bool stream_capturing(hipStream_t st) {
-  if (st == nullptr) return false;
+  if (st == nullptr || st == hipStreamLegacy) return false;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
     (void)hipGetLastError();
@@ -370,47 +399,34 @@ struct RelaxedCapture {
   }
 };
 
-static int split_workspace_acquire_locked(int dev, size_t part_bytes, int ncounters, hipStream_t st, float** ws,
-                                          int** cnt);
-static int capture_workspace_locked(int dev, size_t part_bytes, float** ws);
+// A split launch's workspace; `slot` is locked until split_workspace_release
+// (nullptr for a captured launch: nothing to release).
+struct WsLease {
+  SplitWorkspace* slot = nullptr;
+  float* ws = nullptr;
+  int* cnt = nullptr;
+};
 
-// On SF_OK the workspace lock stays held until split_workspace_release,
-// which the caller must then call (after its launch, whatever that
-// returned); on failure nothing stays locked.  `capturing`: st is being
-// captured (no counters then).
-static int split_workspace_acquire(size_t part_bytes, int ncounters, hipStream_t st, bool capturing, float** ws,
-                                   int** cnt) {
-  int dev = 0;
-  int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
-  if (rc != SF_OK) return rc;
-  g_ws_mu.lock();
-  *cnt = nullptr;
-  rc = capturing ? capture_workspace_locked(dev, part_bytes, ws)
-                 : split_workspace_acquire_locked(dev, part_bytes, ncounters, st, ws, cnt);
-  if (rc != SF_OK) g_ws_mu.unlock();
-  return rc;
-}
-
-static int capture_workspace_locked(int dev, size_t part_bytes, float** ws) {
-  SplitWorkspace& w = g_ws[dev];
-  if (part_bytes > w.capture_bytes) {
-    const size_t want = part_bytes > 2 * w.capture_bytes ? part_bytes : 2 * w.capture_bytes;
-    RelaxedCapture relaxed;
-    void* p = nullptr;
-    const int rc = check_hip(hipMalloc(&p, want), "hipMalloc (capture workspace)");
-    if (rc != SF_OK) return rc;
-    w.capture_base = p;
-    w.capture_bytes = want;
-    w.capture_total += want;
+// The stream's own slot, else one that is free, else the least recently used.
+static SplitWorkspace& pick_slot(DeviceWorkspaces& d, StreamKey key) {
+  SplitWorkspace* best = nullptr;
+  for (SplitWorkspace& w : d.slot) {
+    if (w.owner == key) {
+      best = &w;
+      break;
+    }
+    const bool idle = w.owner == kNoStream;
+    if (best == nullptr || (idle && best->owner != kNoStream) ||
+        (idle == (best->owner == kNoStream) && w.tick < best->tick))
+      best = &w;
   }
-  *ws = static_cast<float*>(w.capture_base);
-  return SF_OK;
+  best->owner = key;
+  best->tick = ++d.tick;
+  return *best;
 }
 
-static int split_workspace_acquire_locked(int dev, size_t part_bytes, int ncounters, hipStream_t st, float** ws,
-                                          int** cnt) {
+static int slot_acquire_locked(SplitWorkspace& w, size_t part_bytes, int ncounters, hipStream_t st, StreamKey key) {
   int rc = SF_OK;
-  SplitWorkspace& w = g_ws[dev];
   if (w.done == nullptr) {
     rc = check_hip(hipEventCreateWithFlags(&w.done, hipEventDisableTiming), "hipEventCreate (split workspace)");
     if (rc != SF_OK) return rc;
@@ -438,37 +454,118 @@ static int split_workspace_acquire_locked(int dev, size_t part_bytes, int ncount
     w.base = p;
     w.part_bytes = pb;
     w.counters = nc;
-    w.used = false;
-  } else if (w.used && w.last != st) {
-    if (w.multi) {
+  } else if (w.used && w.last != key) {
+    if (w.recorded) {
       rc = check_hip(hipStreamWaitEvent(st, w.done, 0), "hipStreamWaitEvent (split workspace)");
     } else {
-      // No event was recorded after the earlier launches: wait for them
-      // once (safe even if their stream has been destroyed since).
+      // No event follows the latest launch: wait for it once (safe even if
+      // its stream has been destroyed since).
+      RelaxedCapture relaxed;
       rc = check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize (split workspace, second stream)");
-      w.multi = true;
     }
     if (rc != SF_OK) return rc;
+    w.multi = w.last != kNoStream;
   }
-  *ws = static_cast<float*>(w.base);
-  *cnt = reinterpret_cast<int*>(static_cast<uint8_t*>(w.base) + w.part_bytes);
   return SF_OK;
 }
 
-// Records the event after the caller's launch (once split launches have
-// come on more than one stream) and releases the lock taken by
-// split_workspace_acquire.
-static int split_workspace_release(hipStream_t st, bool capturing) {
-  std::lock_guard<std::mutex> lk(g_ws_mu, std::adopt_lock);
-  if (capturing) return SF_OK;
+// On SF_OK the caller launches and then calls split_workspace_release,
+// whatever the launch returned; on failure nothing stays locked.  A launch
+// that is being captured takes no counters.
+static int split_workspace_acquire(size_t part_bytes, int ncounters, hipStream_t st, WsLease* lease) {
   int dev = 0;
   int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
   if (rc != SF_OK) return rc;
-  SplitWorkspace& w = g_ws[dev];
-  w.last = st;
+  if (stream_capturing(st)) {
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    DeviceWorkspaces& d = g_ws[dev];
+    if (part_bytes > d.capture_bytes) {
+      const size_t want = part_bytes > 2 * d.capture_bytes ? part_bytes : 2 * d.capture_bytes;
+      RelaxedCapture relaxed;
+      void* p = nullptr;
+      rc = check_hip(hipMalloc(&p, want), "hipMalloc (capture workspace)");
+      if (rc != SF_OK) return rc;
+      d.capture_base = p;
+      d.capture_bytes = want;
+      d.capture_total += want;
+    }
+    lease->ws = static_cast<float*>(d.capture_base);
+    return SF_OK;
+  }
+  const StreamKey key = stream_key(st);
+  SplitWorkspace* w = nullptr;
+  {
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    w = &pick_slot(g_ws[dev], key);
+  }
+  w->mu.lock();
+  rc = slot_acquire_locked(*w, part_bytes, ncounters, st, key);
+  if (rc != SF_OK) {
+    w->mu.unlock();
+    return rc;
+  }
+  lease->slot = w;
+  lease->ws = static_cast<float*>(w->base);
+  lease->cnt = reinterpret_cast<int*>(static_cast<uint8_t*>(w->base) + w->part_bytes);
+  return SF_OK;
+}
+
+// Records the event after the caller's launch (on a buffer that several
+// streams share) and releases the slot.
+static int split_workspace_release(const WsLease& lease, hipStream_t st) {
+  if (lease.slot == nullptr) return SF_OK;
+  SplitWorkspace& w = *lease.slot;
+  std::lock_guard<std::mutex> lk(w.mu, std::adopt_lock);
+  w.last = stream_key(st);
   w.used = true;
+  w.recorded = false;
   if (!w.multi) return SF_OK;
-  return check_hip(hipEventRecord(w.done, st), "hipEventRecord (split workspace)");
+  const int rc = check_hip(hipEventRecord(w.done, st), "hipEventRecord (split workspace)");
+  w.recorded = rc == SF_OK;
+  return rc;
+}
+
+// The devices' workspaces (map nodes stay where they are).
+static std::vector<std::pair<int, DeviceWorkspaces*>> all_workspaces(int device) {
+  std::lock_guard<std::mutex> lk(g_ws_mu);
+  std::vector<std::pair<int, DeviceWorkspaces*>> v;
+  for (auto& kv : g_ws)
+    if (device < 0 || kv.first == device) v.emplace_back(kv.first, &kv.second);
+  return v;
+}
+
+// Before `st` is destroyed: its slots' latest launches are marked by their
+// events (another stream may get the same handle), and the slots are free.
+static void split_workspace_forget(hipStream_t st) {
+  const StreamKey key = stream_key(st);
+  for (auto& dw : all_workspaces(-1))
+    for (SplitWorkspace& w : dw.second->slot) {
+      std::lock_guard<std::mutex> lk(w.mu);
+      if (w.used && w.last == key) {
+        if (!w.recorded) w.recorded = hipEventRecord(w.done, st) == hipSuccess;
+        if (!w.recorded) (void)hipGetLastError();
+        w.last = kNoStream;
+      }
+      std::lock_guard<std::mutex> lk2(g_ws_mu);
+      if (w.owner == key) w.owner = kNoStream;
+    }
+}
+
+// Gives back the device's buffers but the first (current device: `d`'s).
+static void split_workspace_trim(DeviceWorkspaces& d) {
+  for (int i = 1; i < kWsSlots; ++i) {
+    SplitWorkspace& w = d.slot[i];
+    std::lock_guard<std::mutex> lk(w.mu);
+    if (w.base == nullptr || hipDeviceSynchronize() != hipSuccess) continue;
+    (void)hipFree(w.base);
+    w.base = nullptr;
+    w.part_bytes = 0;
+    w.counters = 0;
+    w.used = w.multi = w.recorded = false;
+    w.last = kNoStream;
+    std::lock_guard<std::mutex> lk2(g_ws_mu);
+    w.owner = kNoStream;
+  }
 }
 
 static bool valid_dtype(int d) { return d == SF_F32 || d == SF_F16 || d == SF_BF16; }
@@ -817,10 +914,13 @@ static int gemm_run(int transA, int transB, int64_t M, int64_t N, int64_t K, int
     part_bytes = 0;
   }
   if (part_bytes == 0) return gemm_launch_plan(plan, batch, ab_dtype, c_dtype, st);
-  rc = split_workspace_acquire(part_bytes, counters, st, false, &plan.p.ws, &plan.p.counters);
+  WsLease lease;
+  rc = split_workspace_acquire(part_bytes, counters, st, &lease);
   if (rc != SF_OK) return rc;
+  plan.p.ws = lease.ws;
+  plan.p.counters = lease.cnt;
   rc = gemm_launch_plan(plan, batch, ab_dtype, c_dtype, st);
-  const int rc2 = split_workspace_release(st, false);
+  const int rc2 = split_workspace_release(lease, st);
   return rc != SF_OK ? rc : rc2;
 }
 
@@ -941,14 +1041,12 @@ static int attn_prepare(const char* name, const void* Q, int64_t ldq, int64_t st
 static int attn_wide_run(const AttnShape& a, const AttnMask& m, float scale, sf_dtype dtype, int cus, hipStream_t st) {
   const AttnSplit sp = attn_wide_split_plan(a, cus);
   if (sp.parts == 0) return launch_attention_wide(a, m, scale, dtype, sp, nullptr, st);
-  float* ws = nullptr;
-  int* cnt = nullptr;
-  const bool cap = stream_capturing(st);
+  WsLease lease;
   int rc = split_workspace_acquire((size_t)(sp.items - sp.full) * (size_t)sp.parts * attn_wide_part_bytes(a.D), 0, st,
-                                   cap, &ws, &cnt);
+                                   &lease);
   if (rc != SF_OK) return rc;
-  rc = launch_attention_wide(a, m, scale, dtype, sp, ws, st);
-  const int rc2 = split_workspace_release(st, cap);
+  rc = launch_attention_wide(a, m, scale, dtype, sp, lease.ws, st);
+  const int rc2 = split_workspace_release(lease, st);
   return rc != SF_OK ? rc : rc2;
 }
 
@@ -974,14 +1072,11 @@ int sf_attention_heads(const void* Q, int64_t ldq, int64_t strideQ, int64_t head
     return attn_wide_run(a, AttnMask{nullptr, dtype, 0, 0, 0}, scale, dtype, cus, st);
   const AttnSplit sp = attn_split_plan(a, cus);
   if (sp.parts == 0) return launch_attention(a, scale, dtype, sp, nullptr, st);
-  float* ws = nullptr;
-  int* cnt = nullptr;
-  const bool cap = stream_capturing(st);
-  rc = split_workspace_acquire((size_t)(sp.items - sp.full) * (size_t)sp.parts * kAttnPartBytes, 0, st, cap, &ws,
-                               &cnt);
+  WsLease lease;
+  rc = split_workspace_acquire((size_t)(sp.items - sp.full) * (size_t)sp.parts * kAttnPartBytes, 0, st, &lease);
   if (rc != SF_OK) return rc;
-  rc = launch_attention(a, scale, dtype, sp, ws, st);
-  const int rc2 = split_workspace_release(st, cap);
+  rc = launch_attention(a, scale, dtype, sp, lease.ws, st);
+  const int rc2 = split_workspace_release(lease, st);
   return rc != SF_OK ? rc : rc2;
 }
 
@@ -1086,13 +1181,11 @@ int sf_sum_dim(const void* x, void* out, int64_t outer, int64_t dim_size, int64_
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int S = sum_dim_parts(outer, dim_size, inner, cu_count_current());
   if (S == 1) return launch_sum_dim(x, out, outer, dim_size, inner, in_dtype, out_dtype, nullptr, 1, st);
-  float* ws = nullptr;
-  int* cnt = nullptr;
-  const bool cap = stream_capturing(st);
-  int rc = split_workspace_acquire((size_t)S * (size_t)outer * (size_t)inner * sizeof(float), 0, st, cap, &ws, &cnt);
+  WsLease lease;
+  int rc = split_workspace_acquire((size_t)S * (size_t)outer * (size_t)inner * sizeof(float), 0, st, &lease);
   if (rc != SF_OK) return rc;
-  rc = launch_sum_dim(x, out, outer, dim_size, inner, in_dtype, out_dtype, ws, S, st);
-  const int rc2 = split_workspace_release(st, cap);
+  rc = launch_sum_dim(x, out, outer, dim_size, inner, in_dtype, out_dtype, lease.ws, S, st);
+  const int rc2 = split_workspace_release(lease, st);
   return rc != SF_OK ? rc : rc2;
 }
 
@@ -1392,6 +1485,12 @@ int sf_cache_empty(int device) {
     if (rc != SF_OK) return rc;
     drain_pool(kv.second);
   }
+  for (auto& dw : all_workspaces(device)) {
+    DeviceGuard g;
+    int rc = g.enter(dw.first);
+    if (rc != SF_OK) return rc;
+    split_workspace_trim(*dw.second);
+  }
   return SF_OK;
 }
 
@@ -1410,12 +1509,14 @@ int sf_cache_stats(int device, size_t* pooled_bytes, size_t* live_bytes) {
 
 int sf_workspace_bytes(int device, size_t* bytes) {
   if (bytes == nullptr) return fail(SF_ERR_INVALID_ARG, "sf_workspace_bytes: null pointer");
-  std::lock_guard<std::mutex> lk(g_ws_mu);
   size_t total = 0;
-  for (auto& kv : g_ws) {
-    if (device >= 0 && kv.first != device) continue;
-    if (kv.second.base != nullptr) total += kv.second.part_bytes + (size_t)kv.second.counters * sizeof(int);
-    total += kv.second.capture_total;
+  for (auto& dw : all_workspaces(device)) {
+    for (SplitWorkspace& w : dw.second->slot) {
+      std::lock_guard<std::mutex> lk(w.mu);
+      if (w.base != nullptr) total += w.part_bytes + (size_t)w.counters * sizeof(int);
+    }
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    total += dw.second->capture_total;
   }
   *bytes = total;
   return SF_OK;
@@ -1466,6 +1567,7 @@ int sf_stream_create(void** stream) {
 
 int sf_stream_destroy(void* stream) {
   if (stream == nullptr) return SF_OK;
+  split_workspace_forget((hipStream_t)stream);
   return check_hip(hipStreamDestroy((hipStream_t)stream), "hipStreamDestroy");
 }
 
