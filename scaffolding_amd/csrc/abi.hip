@@ -252,6 +252,19 @@ static int choose_tile16(int64_t M, int64_t N, int64_t K, int64_t batch, bool ve
     if (N > 64 && t256 == cus) return TILE_256x256;
     if (N > 64 && K < 256 && tiles(256, 128) == cus && cfg < 0) return TILE_256x128;
   }
+  if (kvec && !small) {
+    // Operands of 2 GiB and more, past the direct loads' 32-bit offsets: the
+    // register-staged tiles.  300000 x 4096 x 4096 NT 10.9 ms against 11.7
+    // for the 128 x 128 unaligned kernel below, 4096 x 262144 x 5376 11.9
+    // against 13.4, 256 x 300000 x 4096 0.75 against 0.92, 150000 x 4096 x
+    // 8192 NN 12.3 against 12.8 ms.  That kernel stays ahead with at most 128
+    // rows or columns (128 x 300000 x 4096 0.54 against 0.66 ms), with fewer
+    // tiles (its k split: TN 2048 x 2048 x 600000 7.5 against 29.7 ms) and
+    // with an M-contiguous A (TN 4096 x 4096 x 300000 14.7 against 15.1, 5120
+    // x 4096 x 300000 20.9 against 31.8 ms; TT within 6 % either way).
+    if (N <= 64 && tiles(256, 64) >= cus) return TILE_256x64;
+    if (a_kmajor && M > 128 && N > 128 && t256 >= cus) return TILE_256x256;
+  }
   const bool aligned = kvec && small;
   const MidCost* c = aligned ? kMidAligned : (a_kmajor && b_kmajor ? kMidRagged : kMidRaggedMn);
   const int nc = aligned ? (a_kmajor && b_kmajor ? 3 : 2) : 2;
