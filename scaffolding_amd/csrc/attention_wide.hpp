@@ -551,10 +551,8 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
     for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
       for (int db = 0; db < DB; ++db) po[(mb * DB + db) * 64] = o[mb][db];
-      // A row that met no key in this part weighs nothing in the merge; one
-      // that met only NaN scores (no reference either) keeps its NaN sums.
-      const bool none = th[mb] < 0.f && osum[mb][0] == 0.f;
-      pml[mb * 64] = float2{none ? -INFINITY : -nq[mb][0], osum[mb][0]};
+      // a row that met no key in this part weighs nothing in the merge
+      pml[mb * 64] = float2{th[mb] < 0.f ? -INFINITY : -nq[mb][0], osum[mb][0]};
     }
     return;
   }

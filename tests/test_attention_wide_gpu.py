@@ -180,33 +180,3 @@ def test_abi_rules():
     p = P(x.data_ptr)
     assert lib.sf_attention(p, I64(80), I64(0), p, I64(80), I64(0), p, I64(80), I64(0), p, I64(80), I64(0), I64(1),
                             I64(8), I64(8), I64(80), F(0.1), 2, None) == -3
-
-
-@pytest.mark.parametrize("d", [64, 128])
-@pytest.mark.parametrize("masked", [False, True])
-def test_split_parts_of_nan_scores(d, masked):
-    """A key range whose every score is NaN (one part of three, test hook),
-    a NaN query row and an infinite key: NaN wherever the plain softmax is,
-    and nowhere else."""
-    sq, sk = 130, 700
-    rng = np.random.default_rng(d + masked)
-    q, k, v = (rnd(rng, (3, s, d), 1.0, "bfloat16") for s in (sq, sk, sk))
-    k[0, 192:448] = np.nan  # 11 blocks of 64 keys: part 1 is blocks 3 to 6
-    q[1, 7, 3] = np.nan
-    k[2, 50, 5] = np.inf
-    m = None
-    if masked:
-        m = np.zeros((3, sq, sk), np.float32)
-        m[0, :, :192] = -np.inf  # and the first part has no key
-        m[2, 20:, 50] = -np.inf
-    g = cu()
-    g._set_test_hooks(attn_parts=3)
-    try:
-        y = down(g.dev_scaled_dot_product_attention(up(q, "bfloat16"), up(k, "bfloat16"), up(v, "bfloat16"), None,
-                                                    None if m is None else up(m, "float32")))
-    finally:
-        g._set_test_hooks()
-    with np.errstate(invalid="ignore"):
-        s = d ** -0.5 * np.matmul(q.astype(np.float64), np.swapaxes(k, -2, -1).astype(np.float64))
-        y64 = np.matmul(softmax64(s if m is None else s + m), v.astype(np.float64))
-    assert np.array_equal(np.isnan(y), np.isnan(y64))
