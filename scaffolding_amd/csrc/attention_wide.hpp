@@ -125,11 +125,12 @@ __device__ __forceinline__ void attn_special_rows(const AttnWideParams& wp, int6
           }
 #pragma unroll
           for (int u = 0; u < 8; ++u) {
-            n += in[u] ? 1.f : 0.f;
+            const float pu = in[u] ? 1.f : 0.f;  // times V: a NaN or infinite V reaches the row
+            n += pu;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
               const uint32_t w = v[u][e >> 1];
-              acc[e] += in[u] ? Elem<T>::to_f32((uint16_t)(w >> ((e & 1) * 16))) : 0.f;
+              acc[e] = __builtin_fmaf(pu, Elem<T>::to_f32((uint16_t)(w >> ((e & 1) * 16))), acc[e]);
             }
           }
         }

@@ -180,3 +180,25 @@ def test_abi_rules():
     p = P(x.data_ptr)
     assert lib.sf_attention(p, I64(80), I64(0), p, I64(80), I64(0), p, I64(80), I64(0), p, I64(80), I64(0), I64(1),
                             I64(8), I64(8), I64(80), F(0.1), 2, None) == -3
+
+
+def test_non_finite_values_at_keys_without_weight():
+    """Rows whose mask holds only lowest values (or -inf and one of them):
+    P V multiplies every key's V by its weight, so a NaN or infinite V at a
+    key of weight 0 makes its column NaN as in any other row."""
+    rng = np.random.default_rng(12)
+    q, k, v = (rnd(rng, (2, s, 72), 1.0, "float16") for s in (20, 90, 90))
+    v[0, 10, 3] = np.nan
+    v[1, 70, 65] = -np.inf
+    m = np.full((20, 90), LOW, np.float32)
+    m[5:, 10] = -np.inf
+    m[9:, 64:] = -np.inf
+    m[12] = 0.0
+    y = down(cu().dev_scaled_dot_product_attention(up(q, "float16"), up(k, "float16"), up(v, "float16"), None,
+                                                   up(m, "float32")))
+    s = (72 ** -0.5 * np.matmul(q, np.swapaxes(k, -2, -1))).astype(np.float32) + m
+    with np.errstate(invalid="ignore"):
+        y64 = np.matmul(softmax64(s.astype(np.float64)), v.astype(np.float64))
+    ok = np.isfinite(y64)
+    assert np.array_equal(np.isnan(y), np.isnan(y64)) and np.array_equal(y[np.isinf(y64)], y64[np.isinf(y64)])
+    assert np.abs(y[ok] - y64[ok]).max() <= 6 * 2.0 ** -11 * np.abs(v[np.isfinite(v)]).max()
