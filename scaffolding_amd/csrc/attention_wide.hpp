@@ -81,12 +81,13 @@ __device__ __forceinline__ f32x4 mask4(const void* row, int64_t j) {
 }
 
 // Output rows whose every key is masked to -inf or so far down that the mask
-// overflowed in the exponent domain (below about -2e38).  There mask + score
-// is the mask itself in fp32, so the softmax is uniform over the keys that
-// carry the row's largest mask value, and NaN where that is -inf: what
-// softmax(scores + mask) gives.  (A row with a NaN or infinite score is not
-// sent here: its exponents are NaN.)  `rows`: bit i for row q0 + i.  One
-// wave; rows that share one mask row (mR == 0) share the sum.
+// overflowed in the exponent domain (below about -2e38), all scores finite.
+// There mask + score is the mask itself in fp32, so the softmax is uniform
+// over the keys that carry the row's largest mask value, and NaN where that
+// is -inf: what softmax(scores + mask) gives.  (A row with a NaN or +inf
+// score is not sent here: its exponents are NaN; one with a score of -inf
+// goes to attn_exact_rows.)  `rows`: bit i for row q0 + i.  One wave; rows
+// that share one mask row (mR == 0) share the sum.
 template <typename T, int MK>
 __device__ __forceinline__ void attn_special_rows(const AttnWideParams& wp, int64_t b, int64_t h, int q0,
                                                   uint64_t rows) {
@@ -150,14 +151,97 @@ __device__ __forceinline__ void attn_special_rows(const AttnWideParams& wp, int6
   }
 }
 
-// Stores one 16-row block; with a mask, rows whose sum is zero (no key
-// within reach of the exponent domain) are recomputed.
-template <typename T, int DB, int MK>
-__device__ __forceinline__ void attn_wide_store(const AttnWideParams& wp, int64_t b, int64_t h, int q0, int lane,
-                                                const f32x4 (&o)[DB], float l) {
+// Output rows without a key in reach of the exponent domain that met a score
+// of -inf: softmax(scores + mask) V term by term in fp32, scores from global
+// memory: slow, for inputs that hold such values.  One wave.
+template <typename T, int MK>
+__device__ __forceinline__ void attn_exact_rows(const AttnWideParams& wp, int64_t b, int64_t h, int q0,
+                                                uint64_t rows) {
+  constexpr float LN2 = 0.6931471805599453f, LOG2E = 1.4426950408889634f;
   const AttnParams& p = wp.a;
+  const int lane = threadIdx.x & 63;
+  const uint16_t* Kb = static_cast<const uint16_t*>(p.K) + b * p.sK + h * p.hK;
+  const uint16_t* Vb = static_cast<const uint16_t*>(p.V) + b * p.sV + h * p.hV;
+  const float scale = p.scale_log2e * LN2;
+  const bool dok = 2 * lane < p.D;  // lane: columns 2 lane, 2 lane + 1
+  while (rows != 0) {
+    const int r = q0 + __builtin_ctzll(rows);
+    rows &= rows - 1;
+    const uint16_t* qrow = static_cast<const uint16_t*>(p.Q) + b * p.sQ + h * p.hQ + (int64_t)r * p.ldq;
+    const int64_t mo = b * wp.mB + h * wp.mH + (int64_t)r * wp.mR;
+    const void* mrow = MK == 1 ? (const void*)(static_cast<const float*>(wp.mask) + mo)
+                               : (const void*)(static_cast<const uint16_t*>(wp.mask) + mo);
+    auto score = [&](int j) {
+      const uint16_t* krow = Kb + (int64_t)j * p.ldk;
+      float dot = 0.f;
+#pragma nounroll
+      for (int d = 0; d < p.D; d += 8) {
+        const u32x4 qv = *reinterpret_cast<const u32x4*>(qrow + d), kv = *reinterpret_cast<const u32x4*>(krow + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t qw = qv[e], kw = kv[e];
+          dot = __builtin_fmaf(Elem<T>::to_f32((uint16_t)(qw & 0xffffu)), Elem<T>::to_f32((uint16_t)(kw & 0xffffu)), dot);
+          dot = __builtin_fmaf(Elem<T>::to_f32((uint16_t)(qw >> 16)), Elem<T>::to_f32((uint16_t)(kw >> 16)), dot);
+        }
+      }
+      return __builtin_fmaf(dot, scale, mask_at<T, MK>(mrow, j));
+    };
+    float mx = -INFINITY;
+    bool bad = false;
+#pragma nounroll
+    for (int j = lane; j < p.Sk; j += 64) {
+      const float x = score(j);
+      bad |= x != x;
+      mx = fmaxf(mx, x);
+    }
+    mx = wave_max(mx);
+    // NaN scores, +inf (inf - inf) or nothing but -inf
+    bad = __builtin_amdgcn_ballot_w64(bad) != 0 || !(mx > -INFINITY) || mx == INFINITY;
+    float l = 0.f, a0 = 0.f, a1 = 0.f;
+    if (!bad) {
+#pragma nounroll
+      for (int j0 = 0; j0 < p.Sk; j0 += 64) {
+        const int n = p.Sk - j0 < 64 ? p.Sk - j0 : 64;
+        const float pj = lane < n ? __builtin_amdgcn_exp2f((score(j0 + lane) - mx) * LOG2E) : 0.f;
+        l += pj;
+#pragma nounroll
+        for (int u = 0; u < n; ++u) {
+          const float pu = __shfl(pj, u, 64);
+          const uint32_t w =
+              *reinterpret_cast<const uint32_t*>(Vb + (int64_t)(j0 + u) * p.ldv + (dok ? 2 * lane : 0));
+          a0 = __builtin_fmaf(pu, Elem<T>::to_f32((uint16_t)(w & 0xffffu)), a0);
+          a1 = __builtin_fmaf(pu, Elem<T>::to_f32((uint16_t)(w >> 16)), a1);
+        }
+      }
+      l = wave_sum(l);
+    }
+    const float inv = 1.0f / l;  // bad: 0 * inf = NaN
+    if (dok)
+      *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(p.O) + b * p.sO + h * p.hO + (int64_t)r * p.ldo + 2 * lane) =
+          pack2<T>(a0 * inv, a1 * inv);
+  }
+}
+
+// Rows of a 16-row block that need other means than its sums: bit i for row
+// q0 + i.  special: no key within reach (attn_special_rows); exact:
+// attn_exact_rows.  l: the row's sum; low: this lane met a score of -inf.
+__device__ __forceinline__ void attn_odd_rows(const AttnWideParams& wp, int64_t b, int64_t h, int q0, int lane,
+                                              float l, bool low, uint64_t& special, uint64_t& exact) {
+  const bool in = q0 + (lane & 15) < wp.a.Sq;
+  uint64_t lows = __builtin_amdgcn_ballot_w64(low);
+  lows |= lows >> 32;
+  lows |= lows >> 16;
+  const uint64_t zero = __builtin_amdgcn_ballot_w64(in && l == 0.f) & 0xffffull;
+  special = zero & ~lows;
+  exact = zero & lows;
+}
+
+// Stores one 16-row block but the rows in `skip`.
+template <typename T, int DB>
+__device__ __forceinline__ void attn_wide_store(const AttnParams& p, int64_t b, int64_t h, int q0, int lane,
+                                                const f32x4 (&o)[DB], float l, uint64_t skip) {
   const int r = q0 + (lane & 15);
-  if (r < p.Sq) {
+  if (r < p.Sq && ((skip >> (lane & 15)) & 1) == 0) {
     uint16_t* orow = static_cast<uint16_t*>(p.O) + b * p.sO + h * p.hO + (int64_t)r * p.ldo;
     const float inv = 1.0f / l;
 #pragma unroll
@@ -167,10 +251,6 @@ __device__ __forceinline__ void attn_wide_store(const AttnWideParams& wp, int64_
         *reinterpret_cast<u32x2*>(orow + d) =
             u32x2{pack2<T>(o[db][0] * inv, o[db][1] * inv), pack2<T>(o[db][2] * inv, o[db][3] * inv)};
     }
-  }
-  if constexpr (MK != 0) {
-    const uint64_t special = __builtin_amdgcn_ballot_w64(r < p.Sq && l == 0.f) & 0xffffull;
-    if (special != 0) attn_special_rows<T, MK>(wp, b, h, q0, special);
   }
 }
 
@@ -292,6 +372,7 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
 
   f32x4 o[MB][DB], osum[MB], nq[MB];
   float th[MB];  // a row is raised when one of its exponents exceeds this
+  uint32_t low = 0;  // bit mb: a row without a reference met a score of -inf here
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
     osum[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -374,6 +455,15 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
           for (int kc = 0; kc < KC; ++kc) kf[kc] = nk[kc];
         }
       });
+      if constexpr (MK != 0 && !REF) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+          float mn = s[mb][0][0];
+#pragma unroll
+          for (int e = 1; e < 16; ++e) mn = fminf(mn, s[mb][e >> 2][e & 3]);
+          low |= (PRE ? mn : mn * p.scale_log2e) == -INFINITY ? 1u << mb : 0u;
+        }
+      }
       if constexpr (!PRE || !REF) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
@@ -552,14 +642,28 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
     for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
       for (int db = 0; db < DB; ++db) po[(mb * DB + db) * 64] = o[mb][db];
-      // a row that met no key in this part weighs nothing in the merge
-      pml[mb * 64] = float2{th[mb] < 0.f ? -INFINITY : -nq[mb][0], osum[mb][0]};
+      // A row that met no key in this part weighs nothing in the merge; its
+      // sum, zero then, tells whether it met a score of -inf.
+      const bool none = th[mb] < 0.f;
+      const bool lo = none && osum[mb][0] == 0.f && ((low >> mb) & 1) != 0;
+      pml[mb * 64] = float2{none ? -INFINITY : -nq[mb][0], lo ? 1.f : osum[mb][0]};
     }
     return;
   }
+  uint64_t special = 0, exact = 0;
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-    attn_wide_store<T, DB, MK>(wp, b, h, q0 + mb * 16, lane, o[mb], osum[mb][0]);
+  for (int mb = 0; mb < MB; ++mb) {
+    uint64_t sp = 0, ex = 0;
+    if constexpr (MK != 0)
+      attn_odd_rows(wp, b, h, q0 + mb * 16, lane, osum[mb][0], ((low >> mb) & 1) != 0, sp, ex);
+    attn_wide_store<T, DB>(p, b, h, q0 + mb * 16, lane, o[mb], osum[mb][0], sp | ex);
+    special |= sp << (16 * mb);
+    exact |= ex << (16 * mb);
+  }
+  if constexpr (MK != 0) {
+    if (special != 0) attn_special_rows<T, MK>(wp, b, h, q0, special);
+    if (exact != 0) attn_exact_rows<T, MK>(wp, b, h, q0, exact);
+  }
 }
 
 // Merges the parts of split items in part order: one wave per 16 query rows.
@@ -581,6 +685,7 @@ __global__ __launch_bounds__(64) void attn_wide_combine_kernel(AttnWideParams wp
 #pragma unroll 8
   for (int q = 0; q < p.parts; ++q) mmax = fmaxf(mmax, base[(int64_t)q * C::PART + ml_off]);
   float l = 0.f;
+  bool low = false;
   f32x4 o[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -588,13 +693,21 @@ __global__ __launch_bounds__(64) void attn_wide_combine_kernel(AttnWideParams wp
   for (int q = 0; q < p.parts; ++q) {
     const float* pq = base + (int64_t)q * C::PART;
     const float2 ml = *reinterpret_cast<const float2*>(pq + ml_off);
+    // (0 times the sums of a part that met only NaN scores stays NaN)
     const float w = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - mmax);
+    low |= ml.x == -INFINITY && ml.y == 1.f;
     l += w * ml.y;
     const f32x4* po = reinterpret_cast<const f32x4*>(pq + o_off);
 #pragma unroll
     for (int db = 0; db < DB; ++db) o[db] += w * po[db * 64];
   }
-  attn_wide_store<T, DB, MK>(wp, wi.b, wi.h, q0, lane, o, l);
+  uint64_t special = 0, exact = 0;
+  if constexpr (MK != 0) attn_odd_rows(wp, wi.b, wi.h, q0, lane, l, low, special, exact);
+  attn_wide_store<T, DB>(p, wi.b, wi.h, q0, lane, o, l, special | exact);
+  if constexpr (MK != 0) {
+    if (special != 0) attn_special_rows<T, MK>(wp, wi.b, wi.h, q0, special);
+    if (exact != 0) attn_exact_rows<T, MK>(wp, wi.b, wi.h, q0, exact);
+  }
 }
 
 }  // namespace sf

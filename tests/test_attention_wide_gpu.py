@@ -202,3 +202,38 @@ def test_non_finite_values_at_keys_without_weight():
     ok = np.isfinite(y64)
     assert np.array_equal(np.isnan(y), np.isnan(y64)) and np.array_equal(y[np.isinf(y64)], y64[np.isinf(y64)])
     assert np.abs(y[ok] - y64[ok]).max() <= 6 * 2.0 ** -11 * np.abs(v[np.isfinite(v)]).max()
+
+
+def _nonfinite_case(seed, d, dtype):
+    rng = np.random.default_rng(seed)
+    return tuple(rnd(rng, (2, s, d), 1.0, dtype) for s in (40, 203, 203))
+
+
+def _check_rows(q, k, v, scale, m, dtype, parts):
+    g = cu()
+    g._set_test_hooks(attn_parts=parts)
+    try:
+        y = down(g.dev_scaled_dot_product_attention(up(q, dtype), up(k, dtype), up(v, dtype), scale, up(m, "float32")))
+    finally:
+        g._set_test_hooks()
+    with np.errstate(invalid="ignore", over="ignore"):
+        y64 = exact(q, k, v, scale or q.shape[-1] ** -0.5, m)
+    check(y, y64, np.abs(v).max(), dtype)
+
+
+@pytest.mark.parametrize("parts", [0, 3])
+@pytest.mark.parametrize("dtype,d,scale", [("bfloat16", 64, None), ("float16", 128, None), ("bfloat16", 96, 2.0)])
+def test_scores_of_minus_infinity_under_a_mask(dtype, d, scale, parts):
+    """An infinite key gives rows of one sign a score of -inf there.  Where
+    no other key counts the row is NaN, not the average that rows without a
+    key in reach of the mask get; beside lowest-value keys those count."""
+    q, k, v = _nonfinite_case(d, d, dtype)
+    q[:, :, 0] = np.abs(q[:, :, 0]) + 0.5  # so score(key) = -inf
+    k[:, :70, 0] = -np.inf
+    m = np.full((40, 203), -np.inf, np.float32)
+    m[:10, :70] = 0.0    # only -inf scores: NaN
+    m[10:20, :30] = 0.0  # beside lowest-value keys with finite scores: those
+    m[10:20, 100:] = LOW
+    m[20:30, :] = 0.0    # beside ordinary keys
+    m[30:, 20:] = LOW    # lowest-value keys, some of -inf scores
+    _check_rows(q, k, v, scale, m, dtype, parts)
