@@ -151,9 +151,10 @@ __device__ __forceinline__ void attn_special_rows(const AttnWideParams& wp, int6
   }
 }
 
-// Output rows without a key in reach of the exponent domain that met a score
-// of -inf: softmax(scores + mask) V term by term in fp32, scores from global
-// memory: slow, for inputs that hold such values.  One wave.
+// Output rows that the exponent domain cannot hold: a mask value whose
+// product with log2 e overflows upwards, a reference raised far up in one
+// step, or a score of -inf in a row without a key in reach.  softmax(scores + mask) V term by term in fp32, scores
+// from global memory: slow, for inputs that hold such values.  One wave.
 template <typename T, int MK>
 __device__ __forceinline__ void attn_exact_rows(const AttnWideParams& wp, int64_t b, int64_t h, int q0,
                                                 uint64_t rows) {
@@ -224,16 +225,38 @@ __device__ __forceinline__ void attn_exact_rows(const AttnWideParams& wp, int64_
 
 // Rows of a 16-row block that need other means than its sums: bit i for row
 // q0 + i.  special: no key within reach (attn_special_rows); exact:
-// attn_exact_rows.  l: the row's sum; low: this lane met a score of -inf.
+// attn_exact_rows.  l: the row's sum; low: this lane met a score of -inf;
+// far: the row's reference was raised by more than FAR.
+template <typename T, int MK>
 __device__ __forceinline__ void attn_odd_rows(const AttnWideParams& wp, int64_t b, int64_t h, int q0, int lane,
-                                              float l, bool low, uint64_t& special, uint64_t& exact) {
+                                              float l, bool low, bool far, uint64_t& special, uint64_t& exact) {
   const bool in = q0 + (lane & 15) < wp.a.Sq;
   uint64_t lows = __builtin_amdgcn_ballot_w64(low);
   lows |= lows >> 32;
   lows |= lows >> 16;
   const uint64_t zero = __builtin_amdgcn_ballot_w64(in && l == 0.f) & 0xffffull;
   special = zero & ~lows;
-  exact = zero & lows;
+  exact = (zero & lows) | (__builtin_amdgcn_ballot_w64(in && far) & 0xffffull);
+  // NaN sums from a finite mask value past the exponent domain
+  uint64_t nans = __builtin_amdgcn_ballot_w64(in && l != l) & 0xffffull;
+  bool have = false, big = false;
+  while (nans != 0) {
+    const int i = __builtin_ctzll(nans);
+    if (!have || wp.mR != 0) {
+      have = true;
+      const int64_t mo = b * wp.mB + h * wp.mH + (int64_t)(q0 + i) * wp.mR;
+      const void* mrow = MK == 1 ? (const void*)(static_cast<const float*>(wp.mask) + mo)
+                                 : (const void*)(static_cast<const uint16_t*>(wp.mask) + mo);
+      big = false;
+      for (int j = lane; j < wp.a.Sk; j += 64) {
+        const float x = mask_at<T, MK>(mrow, j);
+        big |= x > 2.0e38f && x < INFINITY;
+      }
+      big = __builtin_amdgcn_ballot_w64(big) != 0;
+    }
+    if (big) exact |= 1ull << i;
+    nans &= nans - 1;
+  }
 }
 
 // Stores one 16-row block but the rows in `skip`.
@@ -264,7 +287,7 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
   constexpr int KB = 64;
   constexpr int HB = KB * 128;  // one half of a key block
   constexpr int LPB = 4 * HV;   // direct loads per wave and key block
-  constexpr float THRESH = 8.0f, DEEP = 256.0f, UNSET = -3.0e38f, LOG2E = 1.4426950408889634f;
+  constexpr float THRESH = 8.0f, DEEP = 256.0f, FAR = 65536.0f, UNSET = -3.0e38f, LOG2E = 1.4426950408889634f;
   const AttnParams& p = wp.a;
   __shared__ __attribute__((aligned(1024))) uint8_t sK[NS][HV * HB];
   __shared__ __attribute__((aligned(1024))) uint8_t sV[NS][HV * HB];
@@ -372,7 +395,9 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
 
   f32x4 o[MB][DB], osum[MB], nq[MB];
   float th[MB];  // a row is raised when one of its exponents exceeds this
-  uint32_t low = 0;  // bit mb: a row without a reference met a score of -inf here
+  // bit mb: a row without a reference met a score of -inf here; bit 8 + mb:
+  // a row was raised by more than FAR (see below)
+  uint32_t odd = 0;
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
     osum[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -461,7 +486,7 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
           float mn = s[mb][0][0];
 #pragma unroll
           for (int e = 1; e < 16; ++e) mn = fminf(mn, s[mb][e >> 2][e & 3]);
-          low |= (PRE ? mn : mn * p.scale_log2e) == -INFINITY ? 1u << mb : 0u;
+          odd |= (PRE ? mn : mn * p.scale_log2e) == -INFINITY ? 1u << mb : 0u;
         }
       }
       if constexpr (!PRE || !REF) {
@@ -484,13 +509,14 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
             }
       }
     };
-    // With a mask, a row that has met no key yet or only keys far down (a
-    // large finite mask) has no reference that exponents could be formed
-    // against without losing the scores in its magnitude.
+    // With a mask, a row that has met no key yet or only keys far down or
+    // up (a large finite mask) has no reference that exponents could be
+    // formed against: the scores, rounded in its magnitude as their fp32 sum
+    // with the mask is, would be compared with scores that are not.
     bool deep = false;
     if constexpr (MK != 0) {
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) deep |= th[mb] < 0.f || nq[mb][0] > DEEP;
+      for (int mb = 0; mb < MB; ++mb) deep |= th[mb] < 0.f || fabsf(nq[mb][0]) > DEEP;
       deep = __builtin_amdgcn_ballot_w64(deep) != 0;
     }
     if (deep)
@@ -559,6 +585,11 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
           sub = unset ? (found ? mx : 0.f) : fmaxf(mx, 0.f);
           nm = old - sub;
           corr = unset ? 1.0f : __builtin_amdgcn_exp2f(-sub);
+          // A step that far (a large positive mask after smaller ones): this
+          // block's exponents were rounded against the old reference, the
+          // next blocks' ("deep") will be against the new one, an ulp of
+          // sub apart.
+          if (MK != 0 && sub > FAR) odd |= 256u << mb;
         }
         nq[mb] = f32x4{nm, nm, nm, nm};
         if (found) th[mb] = THRESH;
@@ -643,10 +674,13 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
 #pragma unroll
       for (int db = 0; db < DB; ++db) po[(mb * DB + db) * 64] = o[mb][db];
       // A row that met no key in this part weighs nothing in the merge; its
-      // sum, zero then, tells whether it met a score of -inf.
+      // sum, zero then, tells whether it met a score of -inf.  A sum's sign
+      // tells of a far raise.
       const bool none = th[mb] < 0.f;
-      const bool lo = none && osum[mb][0] == 0.f && ((low >> mb) & 1) != 0;
-      pml[mb * 64] = float2{none ? -INFINITY : -nq[mb][0], lo ? 1.f : osum[mb][0]};
+      float l = osum[mb][0];
+      if (none && l == 0.f && ((odd >> mb) & 1) != 0) l = 1.f;
+      if (((odd >> (8 + mb)) & 1) != 0) l = -l;
+      pml[mb * 64] = float2{none ? -INFINITY : -nq[mb][0], l};
     }
     return;
   }
@@ -655,7 +689,8 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
   for (int mb = 0; mb < MB; ++mb) {
     uint64_t sp = 0, ex = 0;
     if constexpr (MK != 0)
-      attn_odd_rows(wp, b, h, q0 + mb * 16, lane, osum[mb][0], ((low >> mb) & 1) != 0, sp, ex);
+      attn_odd_rows<T, MK>(wp, b, h, q0 + mb * 16, lane, osum[mb][0], ((odd >> mb) & 1) != 0,
+                           ((odd >> (8 + mb)) & 1) != 0, sp, ex);
     attn_wide_store<T, DB>(p, b, h, q0 + mb * 16, lane, o[mb], osum[mb][0], sp | ex);
     special |= sp << (16 * mb);
     exact |= ex << (16 * mb);
@@ -685,7 +720,7 @@ __global__ __launch_bounds__(64) void attn_wide_combine_kernel(AttnWideParams wp
 #pragma unroll 8
   for (int q = 0; q < p.parts; ++q) mmax = fmaxf(mmax, base[(int64_t)q * C::PART + ml_off]);
   float l = 0.f;
-  bool low = false;
+  bool low = false, far = false;
   f32x4 o[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -696,13 +731,14 @@ __global__ __launch_bounds__(64) void attn_wide_combine_kernel(AttnWideParams wp
     // (0 times the sums of a part that met only NaN scores stays NaN)
     const float w = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - mmax);
     low |= ml.x == -INFINITY && ml.y == 1.f;
-    l += w * ml.y;
+    far |= ml.y < 0.f;
+    l += w * fabsf(ml.y);
     const f32x4* po = reinterpret_cast<const f32x4*>(pq + o_off);
 #pragma unroll
     for (int db = 0; db < DB; ++db) o[db] += w * po[db * 64];
   }
   uint64_t special = 0, exact = 0;
-  if constexpr (MK != 0) attn_odd_rows(wp, wi.b, wi.h, q0, lane, l, low, special, exact);
+  if constexpr (MK != 0) attn_odd_rows<T, MK>(wp, wi.b, wi.h, q0, lane, l, low, far, special, exact);
   attn_wide_store<T, DB>(p, wi.b, wi.h, q0, lane, o, l, special | exact);
   if constexpr (MK != 0) {
     if (special != 0) attn_special_rows<T, MK>(wp, wi.b, wi.h, q0, special);

@@ -237,3 +237,25 @@ def test_scores_of_minus_infinity_under_a_mask(dtype, d, scale, parts):
     m[20:30, :] = 0.0    # beside ordinary keys
     m[30:, 20:] = LOW    # lowest-value keys, some of -inf scores
     _check_rows(q, k, v, scale, m, dtype, parts)
+
+
+@pytest.mark.parametrize("parts", [0, 3])
+@pytest.mark.parametrize("dtype,d,scale", [("bfloat16", 64, None), ("float16", 128, None), ("bfloat16", 96, 2.0)])
+def test_large_positive_masks(dtype, d, scale, parts):
+    """Masks up to the largest fp32 value: the sum with the score is rounded
+    to fp32, and rows of one such value are uniform over its keys (scores
+    below 32, half an ulp of 1e9)."""
+    q, k, v = _nonfinite_case(d + 1, d, dtype)
+    if scale:
+        q *= 0.25
+    m = np.zeros((40, 203), np.float32)
+    m[:5] = 1e9
+    m[5:10, 100:] = (1e9 + 62528 * np.arange(5))[:, None]  # small masks before
+    m[10:15, 150:] = -LOW
+    m[15:20] = 3e38
+    m[20:25, 7] = 2.5e38
+    m[25:30, ::3] = 2.5e38
+    m[25:30, 1] = np.nan
+    m[30:35, 64:66] = 2.4e38
+    m[35:, 100] = np.inf  # inf - inf
+    _check_rows(q, k, v, scale, m, dtype, parts)
