@@ -10,40 +10,13 @@ import os
 import numpy as np
 import pytest
 
+from attention_check import HALF_ULP, check, exact, softmax64
 from helpers import cu, down, rnd, up
 
 pytestmark = pytest.mark.gpu
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LOW = float(np.finfo(np.float32).min)
-
-
-def softmax64(s):
-    m = np.max(s, -1, keepdims=True)
-    with np.errstate(invalid="ignore"):
-        e = np.exp(s - m)
-    return e / e.sum(-1, keepdims=True)
-
-
-def exact(q, k, v, scale, mask=None):
-    """fp64, with score + mask rounded to fp32 once as the device's sum is
-    (which decides rows of large finite masks)."""
-    s = scale * np.matmul(q.astype(np.float64), np.swapaxes(k, -2, -1).astype(np.float64))
-    if mask is not None:
-        s = (s.astype(np.float32) + mask.astype(np.float32)).astype(np.float64)
-    return np.matmul(softmax64(s), v.astype(np.float64))
-
-
-def check(y, y64, vmax, dtype):
-    """P and the output are rounded once each, Q once more by the pre-scaled
-    path: exponents move by up to u * sum |q_d k_d| * scale log2 e, about
-    4 u for unit-variance heads, so |error| <= (1 + 4 + 1) u max|v| with u the
-    type's half ulp."""
-    u = {"float16": 2.0 ** -11, "bfloat16": 2.0 ** -8}[dtype]
-    assert np.array_equal(np.isnan(y), np.isnan(y64))
-    ok = ~np.isnan(y64)
-    err = np.abs(y.astype(np.float64) - y64)[ok]
-    assert err.max() <= 6 * u * vmax, err.max()
 
 
 def masks(kind, b, h, sq, sk, rng, dtype):
@@ -80,7 +53,7 @@ def test_wide_heads(dtype, d, shape):
     rng = np.random.default_rng(d + sq + sk)
     q, k, v = (rnd(rng, (bh, s, d), 1.0, dtype) for s in (sq, sk, sk))
     y = down(cu().dev_scaled_dot_product_attention(up(q, dtype), up(k, dtype), up(v, dtype)))
-    check(y, exact(q, k, v, d ** -0.5), np.abs(v).max(), dtype)
+    check(y, exact(q, k, v, d ** -0.5, None, dtype), dtype)
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
@@ -96,26 +69,27 @@ def test_masks(dtype, d, scale, kind, mdtype):
     m = masks(kind, b, h, sq, sk, rng, dtype).astype(np.float32)
     gm = up(m, mdtype or dtype)
     y = down(cu().dev_scaled_dot_product_attention(up(q, dtype), up(k, dtype), up(v, dtype), scale, gm))
-    check(y, exact(q, k, v, scale or d ** -0.5, m), np.abs(v).max(), dtype)
+    check(y, exact(q, k, v, scale or d ** -0.5, m, dtype), dtype)
 
 
 @pytest.mark.parametrize("kind", ["none", "causal", "left-low", "rows"])
 @pytest.mark.parametrize("d", [64, 128])
-def test_split_key_ranges(kind, d):
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_split_key_ranges(kind, d, dtype):
     """Every item in three key ranges (test hook): parts in which a row meets
     no key weigh nothing, rows without any key are finished by the merge."""
     b, h, sq, sk = 2, 2, 130, 700
     rng = np.random.default_rng(d)
-    q, k, v = (rnd(rng, (b, h, s, d), 1.0, "bfloat16") for s in (sq, sk, sk))
-    m = None if kind == "none" else masks(kind, b, h, sq, sk, rng, "bfloat16").astype(np.float32)
+    q, k, v = (rnd(rng, (b, h, s, d), 1.0, dtype) for s in (sq, sk, sk))
+    m = None if kind == "none" else masks(kind, b, h, sq, sk, rng, dtype).astype(np.float32)
     g = cu()
     g._set_test_hooks(attn_parts=3)
     try:
-        y = down(g.dev_scaled_dot_product_attention(up(q, "bfloat16"), up(k, "bfloat16"), up(v, "bfloat16"), None,
+        y = down(g.dev_scaled_dot_product_attention(up(q, dtype), up(k, dtype), up(v, dtype), None,
                                                     None if m is None else up(m, "float32")))
     finally:
         g._set_test_hooks()
-    check(y, exact(q, k, v, d ** -0.5, m), np.abs(v).max(), "bfloat16")
+    check(y, exact(q, k, v, d ** -0.5, m, dtype), dtype)
 
 
 def test_nan_and_inf_scores_reach_their_rows():
@@ -135,6 +109,36 @@ def test_nan_and_inf_scores_reach_their_rows():
     assert np.array_equal(np.isnan(y), np.isnan(y64))
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("masked", [False, True])
+def test_split_parts_of_nan_scores(d, masked):
+    """A key range whose every score is NaN (one part of three, test hook),
+    a NaN query row and an infinite key: NaN wherever the plain softmax is,
+    and nowhere else."""
+    sq, sk = 130, 700
+    rng = np.random.default_rng(d + masked)
+    q, k, v = (rnd(rng, (3, s, d), 1.0, "bfloat16") for s in (sq, sk, sk))
+    k[0, 192:448] = np.nan  # 11 blocks of 64 keys: part 1 is blocks 3 to 6
+    q[1, 7, 3] = np.nan
+    k[2, 50, 5] = np.inf
+    m = None
+    if masked:
+        m = np.zeros((3, sq, sk), np.float32)
+        m[0, :, :192] = -np.inf  # and the first part has no key
+        m[2, 20:, 50] = -np.inf
+    g = cu()
+    g._set_test_hooks(attn_parts=3)
+    try:
+        y = down(g.dev_scaled_dot_product_attention(up(q, "bfloat16"), up(k, "bfloat16"), up(v, "bfloat16"), None,
+                                                    None if m is None else up(m, "float32")))
+    finally:
+        g._set_test_hooks()
+    with np.errstate(invalid="ignore"):
+        s = d ** -0.5 * np.matmul(q.astype(np.float64), np.swapaxes(k, -2, -1).astype(np.float64))
+        y64 = np.matmul(softmax64(s if m is None else s + m), v.astype(np.float64))
+    assert np.array_equal(np.isnan(y), np.isnan(y64))
+
+
 def test_packed_heads_of_80_and_columns_past_d():
     """Heads of 80 read in place from a packed projection (the 96-wide tile
     must not take its neighbour's columns), written side by side."""
@@ -143,7 +147,8 @@ def test_packed_heads_of_80_and_columns_past_d():
     qkv = rnd(rng, (b, n, 3 * h * d), 1.0, "float16")
     y = down(cu().dev_attention_packed(up(qkv, "float16"), h))
     q, k, v = (x.reshape(b, n, h, d).transpose(0, 2, 1, 3) for x in np.split(qkv, 3, -1))
-    check(y, exact(q, k, v, d ** -0.5).transpose(0, 2, 1, 3).reshape(b, n, h * d), np.abs(v).max(), "float16")
+    ref = exact(q, k, v, d ** -0.5, None, "float16")
+    check(y, [x.transpose(0, 2, 1, 3).reshape(b, n, h * d) for x in ref], "float16")
 
 
 @pytest.mark.parametrize("shape", [(0, 4, 16, 16), (2, 0, 16, 16), (2, 3, 0, 16), (2, 3, 16, 0)],
@@ -201,7 +206,8 @@ def test_non_finite_values_at_keys_without_weight():
         y64 = np.matmul(softmax64(s.astype(np.float64)), v.astype(np.float64))
     ok = np.isfinite(y64)
     assert np.array_equal(np.isnan(y), np.isnan(y64)) and np.array_equal(y[np.isinf(y64)], y64[np.isinf(y64)])
-    assert np.abs(y[ok] - y64[ok]).max() <= 6 * 2.0 ** -11 * np.abs(v[np.isfinite(v)]).max()
+    # the weights of keys that count are 1 and exact, but in row 12
+    assert np.abs(y[ok] - y64[ok]).max() <= 6 * HALF_ULP["float16"] * np.abs(v[np.isfinite(v)]).max()
 
 
 def _nonfinite_case(seed, d, dtype):
@@ -217,8 +223,8 @@ def _check_rows(q, k, v, scale, m, dtype, parts):
     finally:
         g._set_test_hooks()
     with np.errstate(invalid="ignore", over="ignore"):
-        y64 = exact(q, k, v, scale or q.shape[-1] ** -0.5, m)
-    check(y, y64, np.abs(v).max(), dtype)
+        ref = exact(q, k, v, scale or q.shape[-1] ** -0.5, m, dtype)
+    check(y, ref, dtype)
 
 
 @pytest.mark.parametrize("parts", [0, 3])
