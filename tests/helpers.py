@@ -48,6 +48,17 @@ def gemm_bound(y64: np.ndarray, absprod: np.ndarray, k: int, dtype: str, act: st
     return (1.0 + 1e-6) * (lip * acc + (out_half_ulp_rel(dtype) + 2e-6) * np.abs(y64)) + 1e-7 + sub
 
 
+def gemm_walk_bound(a64: np.ndarray, b64: np.ndarray, y64: np.ndarray, dtype: str):
+    """For products of independent random terms: the k fp32 roundings are a
+    random walk, 64 sqrt(k) 2^-24 of the terms' 2-norm covers six standard
+    deviations of it ten times over, and the output is rounded once (half an
+    ulp).  Never above gemm_bound."""
+    k = a64.shape[1]
+    walk = 64 * 2.0 ** -24 * np.sqrt(k) * np.sqrt((a64 * a64) @ (b64 * b64))
+    return np.minimum(gemm_bound(y64, np.abs(a64) @ np.abs(b64), k, dtype),
+                      walk + (out_half_ulp_rel(dtype) + 2e-6) * np.abs(y64) + 1e-7)
+
+
 def check_bound(y, y64, bound, what=""):
     err = np.abs(np.asarray(y, np.float64) - y64)
     bad = err > bound
@@ -84,5 +95,5 @@ def rnd(rng, shape, std, dtype):
     return quantize((rng.standard_normal(shape) * std).astype(np.float32), dtype)
 
 
-__all__ = ["ref", "quantize", "up", "down", "gemm_bound", "check_bound", "sample_rows", "rnd",
+__all__ = ["ref", "quantize", "up", "down", "gemm_bound", "gemm_walk_bound", "check_bound", "sample_rows", "rnd",
            "storage", "cu"]

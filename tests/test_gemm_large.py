@@ -9,7 +9,7 @@ import os
 import numpy as np
 import pytest
 
-from helpers import check_bound, cu, gemm_bound, rnd, up
+from helpers import check_bound, cu, gemm_walk_bound, rnd, up
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 I64, P, F = ctypes.c_int64, ctypes.c_void_p, ctypes.c_float
@@ -100,13 +100,7 @@ def test_sampled_outputs(case):
     b = (bh(cols, ks).T if tb else bh(ks, cols)).astype(np.float64)
     got = np.stack([y(int(r))[cols] for r in rows])
     y64 = a @ b
-    # fp32 sums of k random terms: a random walk of k roundings, 64 sqrt(k)
-    # 2^-24 of the terms' 2-norm taken for 6 standard deviations, beside the
-    # output's rounding
-    walk = 64 * 2.0 ** -24 * np.sqrt(k) * np.sqrt((a * a) @ (b * b))
-    bound = np.minimum(gemm_bound(y64, np.abs(a) @ np.abs(b), k, "bfloat16"),
-                       walk + (2.0 ** -8 + 2e-6) * np.abs(y64) + 1e-7)
-    check_bound(got, y64, bound, "%s" % (case,))
+    check_bound(got, y64, gemm_walk_bound(a, b, y64, "bfloat16"), "%s" % (case,))
 
 
 def down_rows(g, lib, gc, m, n):
