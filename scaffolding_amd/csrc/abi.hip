@@ -160,23 +160,41 @@ struct MidCost {
   float tau[4];
   float round, ov0, ov1;
 };
-static const MidCost kMidAligned[] = {
+static constexpr MidCost kMidAligned[] = {
     {TILE_MID_128, 128, 128, 2, {0.63f, 0.90f}, 3.0f, 6.0f, 1.0f},
     {TILE_MID_64, 64, 64, 3, {0.25f, 0.335f, 0.57f}, 2.0f, 1.8f, 0.35f},
     {TILE_MID_32, 32, 64, 3, {0.185f, 0.25f, 0.40f}, 1.5f, 1.2f, 0.2f},
 };
 // Register-staged loads of k-contiguous rows, and of operands with k-rows
 // (two transposing reads a fragment, unaligned k-rows).
-static const MidCost kMidRagged[] = {
+static constexpr MidCost kMidRagged[] = {
     {TILE_RAG_128, 128, 128, 2, {0.9f, 1.5f}, 3.0f, 4.0f, 1.2f},
     {TILE_RAG_64, 64, 64, 4, {0.45f, 0.85f, 1.1f, 1.75f}, 2.0f, 2.0f, 0.3f},
 };
-static const MidCost kMidRaggedMn[] = {
+static constexpr MidCost kMidRaggedMn[] = {
     {TILE_RAG_128, 128, 128, 2, {1.2f, 1.8f}, 3.0f, 4.0f, 1.2f},
     {TILE_RAG_64, 64, 64, 4, {0.9f, 1.6f, 1.9f, 2.4f}, 2.0f, 2.0f, 0.3f},
 };
 constexpr int kMaxSplitMid = 8;
 constexpr float kMidFixed = 5.0f;  // launch, first loads, epilogue
+
+// A split launch is resident together, occ parts a CU, at least two of a
+// tile: its partials and counters fit sf_gemm_noalloc's scratch on 256 CUs.
+template <int N>
+constexpr bool mid_fits_scratch(const MidCost (&t)[N]) {
+  for (int i = 0; i < N; ++i)
+    if ((size_t)t[i].occ * 256 * (size_t)(t[i].bm * t[i].bn) * 4 > kNoallocPartBytes ||
+        (size_t)t[i].occ * 256 / 2 * sizeof(int) > kNoallocCounterBytes)
+      return false;
+  return true;
+}
+static_assert(mid_fits_scratch(kMidAligned) && mid_fits_scratch(kMidRagged) && mid_fits_scratch(kMidRaggedMn),
+              "split parts of the mid-size plans against the fixed scratch");
+// fp32: fewer than 256 tiles of 64 x 64 in at most kMaxSplit32 parts, or at
+// most one 128 x 128 part a CU.
+static_assert(size_t(255) * kMaxSplit32 * (64 * 64 * 4) <= kNoallocPartBytes &&
+                  size_t(256) * (128 * 128 * 4) <= kNoallocPartBytes && 255 * sizeof(int) <= kNoallocCounterBytes,
+              "split parts of the fp32 plans against the fixed scratch");
 
 static float mid_cost(const MidCost& c, int64_t M, int64_t N, int64_t K, int64_t batch, int split, int cus) {
   const int64_t wgs = cdiv(M, c.bm) * cdiv(N, c.bn) * batch * split;

@@ -18,9 +18,10 @@
 // The mask block of the next 64 keys is loaded while P V runs.  Its values
 // go into the score MFMAs' C operand (PRE), so a masked score costs two VALU
 // operations more than an unmasked one.  Rows that have no reference yet, or
-// one far down (a large finite mask so far), form their scores without a
-// reference first ("deep"); rows that meet no key at all are finished by
-// attn_special_rows.
+// one far down or up (a large finite mask so far), form their scores without
+// a reference first ("deep"); rows that meet no key at all are finished by
+// attn_special_rows, those that the exponent domain cannot hold by
+// attn_exact_rows.
 //
 // Bound by VALU issue and MFMA alternating in two waves a SIMD, as
 // attn64_kernel.  Measured (bf16, one MI355X; before: three launches with
@@ -153,11 +154,14 @@ __device__ __forceinline__ void attn_special_rows(const AttnWideParams& wp, int6
 
 // Output rows that the exponent domain cannot hold: a mask value whose
 // product with log2 e overflows upwards, a reference raised far up in one
-// step, or a score of -inf in a row without a key in reach.  softmax(scores + mask) V term by term in fp32, scores
-// from global memory: slow, for inputs that hold such values.  One wave.
+// step, or a score of -inf in a row without a key in reach.  softmax(scores +
+// mask) V term by term in fp32, scores from global memory: slow, for inputs
+// that hold such values.  One wave.  Not inlined: its mere presence in the
+// kernels cost launches of few blocks up to 7 % (4 x 8 heads, 77 x 77, D 128:
+// 8.8 -> 9.4 us; called, 8.8 us).
 template <typename T, int MK>
-__device__ __forceinline__ void attn_exact_rows(const AttnWideParams& wp, int64_t b, int64_t h, int q0,
-                                                uint64_t rows) {
+__device__ __attribute__((noinline)) void attn_exact_rows(const AttnWideParams& wp, int64_t b, int64_t h, int q0,
+                                                          uint64_t rows) {
   constexpr float LN2 = 0.6931471805599453f, LOG2E = 1.4426950408889634f;
   const AttnParams& p = wp.a;
   const int lane = threadIdx.x & 63;
@@ -275,6 +279,13 @@ __device__ __forceinline__ void attn_wide_store(const AttnParams& p, int64_t b, 
             u32x2{pack2<T>(o[db][0] * inv, o[db][1] * inv), pack2<T>(o[db][2] * inv, o[db][3] * inv)};
     }
   }
+}
+
+// The kernel's parameters where the launch put them: what a function that is
+// not inlined can take by reference without a copy in scratch.  (Each kernel
+// here has the one parameter, at the segment's start.)
+__device__ __forceinline__ const AttnWideParams& kernel_params() {
+  return *(const AttnWideParams*)__builtin_amdgcn_kernarg_segment_ptr();
 }
 
 // MK: 0 no mask, 1 an fp32 mask, 2 a mask of type T.  PRE: Q scaled by scale
@@ -485,7 +496,7 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
         for (int mb = 0; mb < MB; ++mb) {
           float mn = s[mb][0][0];
 #pragma unroll
-          for (int e = 1; e < 16; ++e) mn = fminf(mn, s[mb][e >> 2][e & 3]);
+          for (int e = 1; e < 16; ++e) mn = __builtin_elementwise_minimum(mn, s[mb][e >> 2][e & 3]);  // NaN: NaN row
           odd |= (PRE ? mn : mn * p.scale_log2e) == -INFINITY ? 1u << mb : 0u;
         }
       }
@@ -684,20 +695,28 @@ __global__ __launch_bounds__(256, 2) void attn_wide_kernel(AttnWideParams wp) {
     }
     return;
   }
-  uint64_t special = 0, exact = 0;
+  // Waves without an odd row end here, ahead of the code for those.
+  bool any = odd != 0;
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    uint64_t sp = 0, ex = 0;
-    if constexpr (MK != 0)
-      attn_odd_rows<T, MK>(wp, b, h, q0 + mb * 16, lane, osum[mb][0], ((odd >> mb) & 1) != 0,
-                           ((odd >> (8 + mb)) & 1) != 0, sp, ex);
-    attn_wide_store<T, DB>(p, b, h, q0 + mb * 16, lane, o[mb], osum[mb][0], sp | ex);
-    special |= sp << (16 * mb);
-    exact |= ex << (16 * mb);
+  for (int mb = 0; mb < MB; ++mb) any |= !(osum[mb][0] > 0.f);
+  if (MK == 0 || __builtin_expect(__builtin_amdgcn_ballot_w64(any) == 0, 1)) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) attn_wide_store<T, DB>(p, b, h, q0 + mb * 16, lane, o[mb], osum[mb][0], 0);
+    return;
   }
   if constexpr (MK != 0) {
+    uint64_t special = 0, exact = 0;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      uint64_t sp = 0, ex = 0;
+      attn_odd_rows<T, MK>(wp, b, h, q0 + mb * 16, lane, osum[mb][0], ((odd >> mb) & 1) != 0,
+                           ((odd >> (8 + mb)) & 1) != 0, sp, ex);
+      attn_wide_store<T, DB>(p, b, h, q0 + mb * 16, lane, o[mb], osum[mb][0], sp | ex);
+      special |= sp << (16 * mb);
+      exact |= ex << (16 * mb);
+    }
     if (special != 0) attn_special_rows<T, MK>(wp, b, h, q0, special);
-    if (exact != 0) attn_exact_rows<T, MK>(wp, b, h, q0, exact);
+    if (exact != 0) attn_exact_rows<T, MK>(kernel_params(), b, h, q0, exact);
   }
 }
 
@@ -737,12 +756,16 @@ __global__ __launch_bounds__(64) void attn_wide_combine_kernel(AttnWideParams wp
 #pragma unroll
     for (int db = 0; db < DB; ++db) o[db] += w * po[db * 64];
   }
-  uint64_t special = 0, exact = 0;
-  if constexpr (MK != 0) attn_odd_rows<T, MK>(wp, wi.b, wi.h, q0, lane, l, low, far, special, exact);
-  attn_wide_store<T, DB>(p, wi.b, wi.h, q0, lane, o, l, special | exact);
+  if (MK == 0 || __builtin_expect(__builtin_amdgcn_ballot_w64(low || far || !(l > 0.f)) == 0, 1)) {
+    attn_wide_store<T, DB>(p, wi.b, wi.h, q0, lane, o, l, 0);
+    return;
+  }
   if constexpr (MK != 0) {
+    uint64_t special = 0, exact = 0;
+    attn_odd_rows<T, MK>(wp, wi.b, wi.h, q0, lane, l, low, far, special, exact);
+    attn_wide_store<T, DB>(p, wi.b, wi.h, q0, lane, o, l, special | exact);
     if (special != 0) attn_special_rows<T, MK>(wp, wi.b, wi.h, q0, special);
-    if (exact != 0) attn_exact_rows<T, MK>(wp, wi.b, wi.h, q0, exact);
+    if (exact != 0) attn_exact_rows<T, MK>(kernel_params(), wi.b, wi.h, q0, exact);
   }
 }
 

@@ -2,14 +2,20 @@
 // device memory (code under HIP graph capture, tight serving loops,
 // harnesses that forbid hipMalloc).
 //
-// sf_gemm's split plans (the split tail of the 256 x 256 kernel, split-K of
-// small fp32 and 16-bit problems) park fp32 partial tiles and per-tile
-// arrival counters in a per-device workspace that sf_gemm allocates on
-// demand.  This entry point runs exactly the same plans (so its results are
-// bit-identical to sf_gemm's) with that workspace taken from `scratch`, a
-// file-scope device array of SF_NOALLOC_SCRATCH_BYTES that every GPU the
-// library runs on holds until the process ends.  It never calls hipMalloc,
-// hipFree or any allocating routine.
+// sf_gemm's split plans park fp32 partial tiles and per-tile arrival counters
+// in a workspace that sf_gemm allocates on demand.  This entry point runs the
+// same plans (so its results are bit-identical to sf_gemm's on a stream that
+// is not being captured; a captured sf_gemm goes without the split) with that
+// workspace taken from `scratch`, a file-scope device array of
+// SF_NOALLOC_SCRATCH_BYTES that every GPU the library runs on holds until the
+// process ends.  It never calls hipMalloc, hipFree or any allocating routine.
+//
+// The most a plan needs on 256 CUs (checked at compile time in abi.hip where
+// its tables decide it, and on every call below):
+//   256 x 256 kernel     one part a CU of 256 KB: 64 MB, 384 counters
+//   mid-size, unaligned  two resident parts a CU of 64 KB (128 x 128), four
+//                        of 16 KB (64 x 64): 32 MB, 512 counters
+//   fp32                 255 tiles in 8 parts of 16 KB: 32 MB, 255 counters
 //
 // The array's name is a host-side stand-in, not a device address: the
 // first call on a device (with that device current) looks the array up
@@ -25,13 +31,6 @@
 #include "sf_internal.hpp"
 
 namespace sf {
-
-// Largest workspace any sf_gemm plan needs on a 256-CU device: a split
-// plan cuts at most one tile per CU into parts, R * s <= CUs, 256 KB of
-// fp32 partial per part (64 MiB), plus one counter per split tile.
-static constexpr size_t kNoallocPartBytes = size_t(64) << 20;
-static constexpr size_t kNoallocCounterBytes = 4096;
-static_assert(SF_NOALLOC_SCRATCH_BYTES == kNoallocPartBytes + kNoallocCounterBytes, "header and library agree");
 
 static __device__ __align__(256) uint8_t scratch[kNoallocPartBytes + kNoallocCounterBytes];
 

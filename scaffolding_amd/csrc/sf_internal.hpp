@@ -96,6 +96,10 @@ int gemm_prepare(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
                  int64_t strideC, sf_dtype ab_dtype, sf_dtype c_dtype, float alpha, const void* bias,
                  sf_epilogue epi, const void* R, int64_t ldr, int64_t strideR, bool need_c, bool may_split,
                  GemmPlan& plan);
+// sf_gemm_noalloc's fixed scratch: partials, then counters.
+constexpr size_t kNoallocPartBytes = size_t(64) << 20;
+constexpr size_t kNoallocCounterBytes = 4096;
+static_assert(SF_NOALLOC_SCRATCH_BYTES == kNoallocPartBytes + kNoallocCounterBytes, "header and library agree");
 // The split plan's workspace: fp32 partials (*part_bytes, 0 without a
 // split) followed by *counters ints that must be zero at launch.
 void gemm_split_needs(const GemmPlan& plan, size_t* part_bytes, int* counters);
