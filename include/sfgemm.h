@@ -85,9 +85,9 @@ int sf_version(void);
 /* Test hooks: force plans the planner would not pick; none of them may
  * change a result.  No counterpart in the reference; for the library's own
  * tests only (the library never reads them from the environment).
- *   xcd_shift   0..7: each part of a persistent split tile expects the XCD
- *               this many places from its own (0: off), so every part
- *               takes the agent-scope fallback hand-off;
+ *   xcd_shift   0..7: each part of a persistent or mid-size split tile
+ *               expects the XCD this many places from its own (0: off), so
+ *               every part takes the agent-scope fallback hand-off;
  *   split_spins 0..256 caps how long a split part waits for the others
  *               (0: the last part sums every slice); -1: the built-in bound;
  *   attn_parts  0, or 2..16: split every fused-attention work item into
@@ -269,8 +269,10 @@ int sf_attention_heads(const void* Q, int64_t ldq, int64_t strideQ, int64_t head
  * of dtype `dtype` or F32 at its natural alignment; NULL for none (the
  * mask_* arguments are then ignored).  -inf entries drop a key; a row of
  * -inf only gives NaN and a row of the type's lowest value only gives the
- * mean of V, as softmax(scores + mask) does.  fp32 scores, mask sum and
- * softmax.  D a multiple of 8 up to 128; the other rules and errors are
+ * mean of V, as softmax(scores + mask) does.  fp32 scores, mask sum (formed
+ * in units of ln 2, so sums with a large finite mask are rounded to 1.44
+ * times the usual step at most) and softmax; Q is rounded once more where
+ * sf_attention rounds it (scale * log2(e) <= 1).  D a multiple of 8 up to 128; the other rules and errors are
  * sf_attention_heads'.  Replaces the masked branch of
  * scaled_dot_product_attention (nn/functional.py:339-347) as well. */
 int sf_attention_masked(const void* Q, int64_t ldq, int64_t strideQ, int64_t headQ,

@@ -44,6 +44,10 @@ static int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 int check_launch(const char* what) { return check_hip(hipGetLastError(), what); }
 
+// A plan's name gives the tile, not the kernel family, which follows from the
+// types: a 16-bit "128x128", "64x64" or "generic" tile with a 16-bit output
+// is gemm16mid_kernel's, with an fp32 output gemm16_kernel's; an fp32 one is
+// gemm32dma_kernel's where the name says "lds-dma", else gemm32_kernel's.
 const char* tile_name(int cfg) {
   switch (cfg) {
     case TILE_256x256: return "gemm tile 256x256";
@@ -151,10 +155,11 @@ static int cu_count_current() {
 // in between, one round of tau[occ - 1] for every further occ workgroups);
 // a further round also costs `round` (its prologue and epilogue), and a
 // split ov0 + ov1 * parts (partials and their sum).  Fitted to sweeps on one
-// MI355X of 133 aligned problems (M 24-6400, N 640-11008, K 104-7680, NT, NN
-// and TN): the plan the estimate picks is on average 1.6 % slower than the
-// fastest one measured, at worst 16 %; 29 unaligned ones: 2.7 %, at worst
-// 17 %.
+// MI355X.  Checked there on 58 problems drawn from M 24-6400, N 640-11008, K
+// 104-7680, NT, NN and TN: the plan the estimate picks takes on average 2.0 %
+// longer than the fastest one measured where rows are aligned (41 problems,
+// at worst 24 %: 235 x 1072 x 4336 NT), 1.3 % where they are not (16
+// problems, at worst 6 %).
 struct MidCost {
   int cfg, bm, bn, occ;
   float tau[4];
@@ -254,9 +259,13 @@ static int choose_tile16(int64_t M, int64_t N, int64_t K, int64_t batch, bool ve
     if (k_ok && N > 64 && M > 64) {
       if (t256 >= cus) return TILE_NT_BIG;
       const bool can_split = may_split && batch == 1 && K >= 1024 && 16 * t256 >= cus;
-      // TT, TN with a ragged K whose split tiles fill the CUs exactly, and
-      // parts with more CUs than the estimates below were fitted on keep the
-      // split of the 256 x 256 kernel.
+      // Left to the split of the 256 x 256 kernel, as before the mid-size
+      // kernels (tests/test_abi_cpu.py pins such plans): TT; devices with
+      // more CUs than the estimates were fitted on; TN with a K that is no
+      // multiple of 128 and a tile count that divides the CUs.  The last is
+      // not the faster choice: TN 1920 x 1920 x 1350 47.7 us against 19.1
+      // on 128 x 128 tiles, 1000 x 1000 x 1112 47.1 against 10.0, 1920 x
+      // 1920 x 4000 61.9 against 42.8.
       if (can_split && (tt || cus > 256 || (K % 128 != 0 && 2 * t256 <= cus && cus % t256 == 0))) return TILE_NT_BIG;
       if (tt ? 2 * t256 >= cus : 4 * t256 >= cus) {
         best = big_cost(t256, K, can_split, cus);
@@ -265,8 +274,10 @@ static int choose_tile16(int64_t M, int64_t N, int64_t K, int64_t batch, bool ve
     }
     if (N <= 64 && tiles(256, 64) >= cus) return TILE_256x64;
     // Exactly one 256 x 256 tile per CU, or with K < 256 one 256 x 128: the
-    // register-staged tiles.  (The 128 x 128 kernel below is the faster one there too, 15.9
-    // against 24.3 us at 4096 x 4096 x 192; the suite pins these plans.)
+    // register-staged tiles (tests/test_abi_cpu.py and test_gemm_gpu.py pin
+    // these plans).  Not the faster choice either: 4096 x 4096 x 192 NT 23.3
+    // us against 14.3 on the 128 x 128 kernel below, x 4000 NN 152 against
+    // 126, 2048 x 4096 x 136 NT 11.7 against 9.1.
     if (N > 64 && t256 == cus) return TILE_256x256;
     if (N > 64 && K < 256 && tiles(256, 128) == cus && cfg < 0) return TILE_256x128;
   }
@@ -734,7 +745,7 @@ int gemm_prepare(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
                      (strideA % 8 == 0) && (strideB % 8 == 0) &&
                      (a_kmajor || M % 8 == 0) && (b_kmajor || N % 8 == 0);
     // The LDS-DMA kernels address each operand (M or K rows of lda) with
-    // 32-bit byte offsets; larger ones take the register-staged loads.
+    // 32-bit byte offsets; larger ones take register-staged loads.
     const bool small = (a_kmajor ? M : K) * lda * 2 < (int64_t(1) << 31) &&
                        (b_kmajor ? N : K) * ldb * 2 < (int64_t(1) << 31);
     plan.fp32 = false;
@@ -990,7 +1001,7 @@ int sf_gemm_plan(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
   char extra[64] = "";
   if (!plan.noop && plan.p.split > 0)
     snprintf(extra, sizeof(extra), "%s split%s %dx%d", plan.p.persist > 0 ? " persistent" : "",
-             split_optional(plan.cfg) ? "" : "-tail",
+             split_whole(plan.cfg) ? "" : "-tail",
              plan.p.tiles_m * plan.p.tiles_n - plan.p.full_tiles, plan.p.split);
   else if (!plan.noop && plan.p.persist > 0)
     snprintf(extra, sizeof(extra), " persistent");

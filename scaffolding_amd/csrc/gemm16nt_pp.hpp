@@ -45,8 +45,8 @@
 // read touches over distinct banks (0 SQ_LDS_BANK_CONFLICT, measured).
 // Columns past M or N read neighbouring data or, past the buffer's end,
 // zeros; their products only reach unstored outputs.  With both operands
-// M/N-contiguous, K may be any multiple of 8: k-rows past K lie beyond both
-// buffers' bounds and read as zeros, so they add nothing.
+// M/N-contiguous, any K will do: k-rows past K lie beyond both buffers'
+// bounds and read as zeros, so they add nothing.
 //
 // Schedule per slice t (group 0 between barriers 2t and 2t+1, group 1 one
 // barrier later): at even t each wave issues its loads of pair t/2 + 1 into

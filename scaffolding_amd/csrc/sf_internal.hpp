@@ -63,8 +63,8 @@ enum TileCfg {
   TILE32_RAG_SPLIT = 20  // as TILE32_DMA_SPLIT
 };
 const char* tile_name(int cfg);
-// Plans whose split may be left out (the unsplit kernel is the same one).
-inline bool split_optional(int cfg) { return (cfg >= TILE_MID_128 && cfg <= TILE_RAG_64) || cfg == TILE32_RAG_SPLIT; }
+// Plans that sf_gemm_plan calls "split" rather than "split-tail".
+inline bool split_whole(int cfg) { return (cfg >= TILE_MID_128 && cfg <= TILE_RAG_64) || cfg == TILE32_RAG_SPLIT; }
 inline bool is_mid(int cfg) { return cfg >= TILE_MID_128 && cfg <= TILE_RAG_64; }
 
 // One GEMM launch: batch entries [0, batch) of p, grid.y <= 65535 per call.

@@ -208,8 +208,8 @@ def test_dispatch_for_config_shapes():
         == "gemm tile 64x64 lds-dma fp32 split-tail 20x8"
     assert plan(M=1000, N=900, K=100, lda=100, ldb=100, ldc=900, dtype="float32") == "gemm tile 64x64 fp32"
     assert plan(M=300, N=260, K=1000, lda=1000, ldb=1000, ldc=260, dtype="float32") == "gemm small 16x32 fp32"
-    # backward GEMMs: dW = dY^T X (A stored K x M) takes the register-staged
-    # tiles, never the LDS-DMA or skinny kernels; dX = dY W is NN
+    # backward GEMMs: dW = dY^T X (A stored K x M, TN), dX = dY W (NN); the
+    # skinny kernels take neither
     assert plan(transA=1, transB=0, M=1920, N=7680, K=17776, lda=1920, ldb=7680, ldc=7680) \
         == "gemm tn 256x256 lds-dma 16-bit"
     assert plan(transA=1, transB=0, M=1920, N=1920, K=17776, lda=1920, ldb=1920, ldc=1920) \
@@ -233,7 +233,7 @@ def test_dispatch_for_config_shapes():
     assert plan(transA=1, transB=1, M=16, N=11008, ldc=11008, lda=16) == "gemm tile 64x64 16-bit"
     assert plan(transA=1, transB=0, M=4092, lda=4092).startswith("gemm tile generic")
     assert plan(transA=1, transB=0, dtype="float32").startswith("gemm tile 128x128 fp32")
-    # unaligned operands fall back to the bounds-checked kernel
+    # operands off 16-byte alignment: gemm16mid_kernel's register-staged loads
     assert plan(K=4095, lda=4095, ldb=4095).startswith("gemm tile generic")
     assert plan(ptr_a=258).startswith("gemm tile generic")
 
