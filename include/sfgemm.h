@@ -130,10 +130,12 @@ int sf_set_test_hooks(int xcd_shift, int split_spins, int attn_parts);
  * M, N or batch == 0 is a no-op; K == 0 writes epi(0 (+ bias)).
  * The call is asynchronous on `stream`.  Some plans split tiles along k and
  * pass fp32 partials through a workspace, allocated on a stream's first use
- * of one (see sf_workspace_bytes, sf_gemm_noalloc).  On a stream that is being captured every problem
- * runs without a split: the call allocates nothing and its graph holds no
- * library memory, so replays need no ordering against other calls.  (A sum
- * that the eager call splits may differ there in its last bits.) */
+ * of one (see sf_workspace_bytes, sf_gemm_noalloc).  On a stream that is
+ * being captured every problem runs without a split: the call allocates
+ * nothing and its graph holds no library memory, so replays need no ordering
+ * against other calls.  So does a call for whose workspace no device memory
+ * is left.  (A sum that is split otherwise may differ there in its last
+ * bits.) */
 int sf_gemm(int transA, int transB,
             int64_t M, int64_t N, int64_t K, int64_t batch,
             const void* A, int64_t lda, int64_t strideA,

@@ -947,23 +947,26 @@ static int gemm_run(int transA, int transB, int64_t M, int64_t N, int64_t K, int
   size_t part_bytes = 0;
   int counters = 0;
   gemm_split_needs(plan, &part_bytes, &counters);
-  if (part_bytes > 0 && stream_capturing(st)) {
-    // A graph may not hold the shared workspace (see SplitWorkspace): the
-    // best plan without a split, nothing allocated or waited for.
+  if (part_bytes > 0) {
+    // A graph may not hold the shared workspace (see SplitWorkspace), and no
+    // memory may be left for it: the best plan without a split then.
+    if (!stream_capturing(st)) {
+      WsLease lease;
+      rc = split_workspace_acquire(part_bytes, counters, st, &lease);
+      if (rc == SF_OK) {
+        plan.p.ws = lease.ws;
+        plan.p.counters = lease.cnt;
+        rc = gemm_launch_plan(plan, batch, ab_dtype, c_dtype, st);
+        const int rc2 = split_workspace_release(lease, st);
+        return rc != SF_OK ? rc : rc2;
+      }
+      if (rc != SF_ERR_OOM) return rc;
+    }
     rc = gemm_prepare(transA, transB, M, N, K, batch, A, lda, strideA, B, ldb, strideB, C, ldc, strideC, ab_dtype,
                       c_dtype, alpha, bias, epi, R, ldr, strideR, true, false, plan);
     if (rc != SF_OK) return rc;
-    part_bytes = 0;
   }
-  if (part_bytes == 0) return gemm_launch_plan(plan, batch, ab_dtype, c_dtype, st);
-  WsLease lease;
-  rc = split_workspace_acquire(part_bytes, counters, st, &lease);
-  if (rc != SF_OK) return rc;
-  plan.p.ws = lease.ws;
-  plan.p.counters = lease.cnt;
-  rc = gemm_launch_plan(plan, batch, ab_dtype, c_dtype, st);
-  const int rc2 = split_workspace_release(lease, st);
-  return rc != SF_OK ? rc : rc2;
+  return gemm_launch_plan(plan, batch, ab_dtype, c_dtype, st);
 }
 
 int sf_gemm(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_t batch, const void* A,

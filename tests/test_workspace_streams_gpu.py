@@ -4,7 +4,10 @@ their sums stay what they are on one stream."""
 from __future__ import annotations
 
 import ctypes
+import json
 import os
+import subprocess
+import sys
 import threading
 
 import numpy as np
@@ -156,3 +159,43 @@ def test_eager_split_call_beside_a_capture():
     hip.hipGraphDestroy(graph)
     for s in streams:
         lib.sf_stream_destroy(s)
+
+
+def test_no_memory_left_for_a_workspace():
+    """A split plan runs unsplit where its workspace cannot be allocated."""
+    r = subprocess.run([sys.executable, os.path.join(ROOT, "tests", "low_memory_process.py")], capture_output=True,
+                       text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+    out = json.loads(r.stdout.strip().splitlines()[-1])
+    assert out["rcs"] == [0, 0, 0] and out["ws"] == 0 and out["held"] > 0 and out["worst"] <= 1.0, out
+
+
+def test_per_thread_streams():
+    """hipStreamPerThread is another stream in every thread: split calls on
+    it from several threads keep apart."""
+    g, lib = cu(), _lib()
+    ops = [_operands(20 + i) for i in range(3)]
+    want, outs = [], [g.empty((M, N), g.BFLOAT16) for _ in range(3)]
+    for x, w in ops:
+        out = g.empty((M, N), g.BFLOAT16)
+        assert _gemm(lib, x, w, out, None) == 0
+        want.append(down(out))
+    g.device_synchronize()
+    errors = []
+
+    def worker(i):
+        for _ in range(40):
+            rc = _gemm(lib, *ops[i], outs[i], P(2))
+            if rc != 0:
+                errors.append(rc)
+        lib.sf_stream_synchronize(P(2))
+
+    ts = [threading.Thread(target=worker, args=(i,)) for i in range(3)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    g.device_synchronize()
+    assert not errors
+    for out, y in zip(outs, want):
+        assert np.array_equal(down(out), y)
