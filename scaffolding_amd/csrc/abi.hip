@@ -397,15 +397,16 @@ struct SplitWorkspace {
 };
 struct DeviceWorkspaces {
   SplitWorkspace slot[kWsSlots];
-  uint64_t tick = 0;
+  uint64_t tick = 0;  // this and the rest under g_ws_mu
   void* capture_base = nullptr;
   size_t capture_bytes = 0;  // of the newest capture buffer
   size_t capture_total = 0;  // of all of them
 };
-// The map, slot owners and ticks, capture buffers.  Never held while a
-// slot's lock is taken.
+// Slot owners and ticks, capture buffers.  Never held while a slot's lock is
+// taken.
 static std::mutex g_ws_mu;
-static std::unordered_map<int, DeviceWorkspaces> g_ws;
+constexpr int kWsDevices = 64;
+static DeviceWorkspaces g_ws[kWsDevices];  // by device ordinal
 
 // A stream's identity: its handle, but hipStreamPerThread names another
 // stream in every thread and hipStreamLegacy the null one.
@@ -518,9 +519,10 @@ static int split_workspace_acquire(size_t part_bytes, int ncounters, hipStream_t
   int dev = 0;
   int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
   if (rc != SF_OK) return rc;
+  if (dev < 0 || dev >= kWsDevices) return fail(SF_ERR_UNSUPPORTED, "split workspace: device ordinal %d above 63", dev);
+  DeviceWorkspaces& d = g_ws[dev];
   if (stream_capturing(st)) {
     std::lock_guard<std::mutex> lk(g_ws_mu);
-    DeviceWorkspaces& d = g_ws[dev];
     if (part_bytes > d.capture_bytes) {
       const size_t want = part_bytes > 2 * d.capture_bytes ? part_bytes : 2 * d.capture_bytes;
       RelaxedCapture relaxed;
@@ -538,7 +540,7 @@ static int split_workspace_acquire(size_t part_bytes, int ncounters, hipStream_t
   SplitWorkspace* w = nullptr;
   {
     std::lock_guard<std::mutex> lk(g_ws_mu);
-    w = &pick_slot(g_ws[dev], key);
+    w = &pick_slot(d, key);
   }
   w->mu.lock();
   rc = slot_acquire_locked(*w, part_bytes, ncounters, st, key);
@@ -567,21 +569,12 @@ static int split_workspace_release(const WsLease& lease, hipStream_t st) {
   return rc;
 }
 
-// The devices' workspaces (map nodes stay where they are).
-static std::vector<std::pair<int, DeviceWorkspaces*>> all_workspaces(int device) {
-  std::lock_guard<std::mutex> lk(g_ws_mu);
-  std::vector<std::pair<int, DeviceWorkspaces*>> v;
-  for (auto& kv : g_ws)
-    if (device < 0 || kv.first == device) v.emplace_back(kv.first, &kv.second);
-  return v;
-}
-
 // Before `st` is destroyed: its slots' latest launches are marked by their
 // events (another stream may get the same handle), and the slots are free.
 static void split_workspace_forget(hipStream_t st) {
   const StreamKey key = stream_key(st);
-  for (auto& dw : all_workspaces(-1))
-    for (SplitWorkspace& w : dw.second->slot) {
+  for (DeviceWorkspaces& d : g_ws)
+    for (SplitWorkspace& w : d.slot) {
       std::lock_guard<std::mutex> lk(w.mu);
       if (w.used && w.last == key) {
         if (!w.recorded) w.recorded = hipEventRecord(w.done, st) == hipSuccess;
@@ -591,6 +584,15 @@ static void split_workspace_forget(hipStream_t st) {
       std::lock_guard<std::mutex> lk2(g_ws_mu);
       if (w.owner == key) w.owner = kNoStream;
     }
+}
+
+// Whether the device holds a buffer beside the first.
+static bool split_workspace_extra(DeviceWorkspaces& d) {
+  for (int i = 1; i < kWsSlots; ++i) {
+    std::lock_guard<std::mutex> lk(d.slot[i].mu);
+    if (d.slot[i].base != nullptr) return true;
+  }
+  return false;
 }
 
 // Gives back the device's buffers but the first (current device: `d`'s).
@@ -1530,12 +1532,13 @@ int sf_cache_empty(int device) {
     if (rc != SF_OK) return rc;
     drain_pool(kv.second);
   }
-  for (auto& dw : all_workspaces(device)) {
-    DeviceGuard g;
-    int rc = g.enter(dw.first);
-    if (rc != SF_OK) return rc;
-    split_workspace_trim(*dw.second);
-  }
+  for (int dev = 0; dev < kWsDevices; ++dev)
+    if ((device < 0 || dev == device) && split_workspace_extra(g_ws[dev])) {
+      DeviceGuard g;
+      int rc = g.enter(dev);
+      if (rc != SF_OK) return rc;
+      split_workspace_trim(g_ws[dev]);
+    }
   return SF_OK;
 }
 
@@ -1555,13 +1558,14 @@ int sf_cache_stats(int device, size_t* pooled_bytes, size_t* live_bytes) {
 int sf_workspace_bytes(int device, size_t* bytes) {
   if (bytes == nullptr) return fail(SF_ERR_INVALID_ARG, "sf_workspace_bytes: null pointer");
   size_t total = 0;
-  for (auto& dw : all_workspaces(device)) {
-    for (SplitWorkspace& w : dw.second->slot) {
+  for (int dev = 0; dev < kWsDevices; ++dev) {
+    if (device >= 0 && dev != device) continue;
+    for (SplitWorkspace& w : g_ws[dev].slot) {
       std::lock_guard<std::mutex> lk(w.mu);
       if (w.base != nullptr) total += w.part_bytes + (size_t)w.counters * sizeof(int);
     }
     std::lock_guard<std::mutex> lk(g_ws_mu);
-    total += dw.second->capture_total;
+    total += g_ws[dev].capture_total;
   }
   *bytes = total;
   return SF_OK;
